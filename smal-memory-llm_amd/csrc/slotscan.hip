@@ -14,16 +14,17 @@
 //
 // A hard write changes exactly one row (kvu/slotkern_kvu.py:8-13), and with the address detached the
 // key/value gradient recursion depends only on WHICH row was written.  The work therefore splits into
-//   chain_fwd  one workgroup per chain, sequential in t: keys + occupancy, the argmax address, the undo log
-//              (row, old key row, old occupancy) and the key snapshots;
-//   rows_fwd   parallel over rows: replays each row's value from the address log, value snapshots;
+//   chain_fwd  one workgroup per chain, sequential in t: keys + occupancy, the argmax address, the log (row, old
+//              occupancy, cosines);
+//   rows_fwd   parallel over rows: replays each row's key and value from the address log, the snapshots and the
+//              undo log (old key and value rows);
 //   rows_bwd   parallel over rows, reverse in t: undoes rows from the log, runs dK/dV, emits dk, dv and
 //              Dn[t, n] = <k_t - K_n, dK_n> + <v_t - V_n, dV_n>;
 //   chain_bwd  one workgroup per chain, reverse in t: undoes keys + occupancy, rebuilds the soft address
 //              and runs its adjoint: dgate, dq, per-token dfr, and per-chain dtemp / scalar-dfr partials
 //              that a fixed-order reduction (reduce_parts) sums -- no float atomics anywhere.
 //
-// gfx950 mapping of the chain kernels.  A chain workgroup is 192 lanes = 3 waves = 12 row groups of 16
+// gfx950 mapping of chain_fwd_reg and chain_bwd (chain_fwd and chain_bwd_w: at the kernels).  A chain workgroup is 192 lanes = 3 waves = 12 row groups of 16
 // lanes (one DPP row each); a row group holds P slot rows (P = 16 at N <= 192), lane c keeping elements
 // {4c..4c+3, 64+4c..} of every one of them, in the same register order in every lane (so the written
 // row's register index is wave-uniform and the update never diverges).  The per-step dot products
@@ -46,6 +47,7 @@ typedef uint64_t u64;
 typedef uint32_t u32;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 #define SLOT_CT 16          // tokens per staged chunk
 #define CHAIN_WAVES 3
@@ -228,15 +230,13 @@ template <int P> __device__ __forceinline__ int row_of_lane(int wave, int lane) 
 struct ChainFwdArgs {
     const void* q; const void* k; const float* gate; const float* fr; const float* temp;
     const float* k0; const float* o0;
-    float* kbuf; int32_t* am; float* kold; float* oold; float* cslog; float* kfin; float* ofin;
-    int T, H, N, G, NB; float eps; int frt, occb;
-    int ts, te;                                          // steps [ts, te) of the T-long sequence; ts % G == 0
-    // the writer-epilogue emission (all NULL: fp32 kbuf): bf16 key copies, kinv and valid per snapshot row
-    bf16_t* kbm; float* kinvm; uint8_t* validm;
-    // chain (b, h) of k0 and kfin is slab b * k0bs + h (kfbs): H for (B*H, N, D) carries; NB * H where a chunk
-    // of the pipeline starts from (ends in) the key snapshot of its first (next) block.  skip0: that first
-    // snapshot is already written (by the previous chunk), so this chunk does not store it.
-    int k0bs, kfbs, skip0;
+    int32_t* am; float* oold; float* cslog; float* kfin; float* ofin;
+    int T, H, N; float eps; int frt, occb;
+    int ts, te;                                          // steps [ts, te) of the T-long sequence
+    // chain_fwd_reg: the fp32 snapshots and the old key rows it writes, and, as RowsFwdArgs, the slabs it starts
+    // from and ends in
+    float* kbuf; float* kold;
+    int G, NB, k0bs, kfbs, skip0;
 };
 
 // Wave-local LDS ordering: lanes of one wave exchange data through LDS (DS instructions of a wave execute
@@ -260,18 +260,6 @@ __device__ __forceinline__ void st_slice_at(float* base, u32 boff, const float* 
     }
 }
 
-// The same slice as bf16 (the writer epilogue's cast, round to nearest even): 8 bytes per 4 elements
-template <int EPL>
-__device__ __forceinline__ void st_slice_bf_at(bf16_t* base, u32 boff, const float* s) {
-    char* p = reinterpret_cast<char*>(base) + boff;
-#pragma unroll
-    for (int jj = 0; jj < EPL / 4; jj++) {
-        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-        const u32x2 r = {pack_bf16x2(s[4 * jj], s[4 * jj + 1]), pack_bf16x2(s[4 * jj + 2], s[4 * jj + 3])};
-        __builtin_nontemporal_store(r, reinterpret_cast<u32x2*>(p + 128 * jj));
-    }
-}
-
 // Wave max of an ordered key (fkey), at every lane: integer max needs no NaN canonicalisation, so each
 // DPP stage is one v_max_u32 with a DPP source.
 __device__ __forceinline__ u32 wavemax_key(u32 v) {
@@ -285,9 +273,15 @@ __device__ __forceinline__ u32 wavemax_key(u32 v) {
     return max(r[0], r[1]);
 }
 
-// The sequential key chain, windowed over the staged 16-step chunks.
+// The key chain with its keys in registers, which also writes the fp32 key snapshots.  It serves the fp32 contract
+// where the chains are more than one round of chain_fwd's workgroups (below) and the forward runs as the chunk
+// pipeline: the pipeline is then bound by its snapshot bytes, and this kernel, half of a CU's registers a
+// workgroup, holds every chain at once and writes the keys' half of them while it steps, in the first chunk
+// too, where the replay has nothing to do yet.  B 64, T 1024, H 6, N 192, D 128, forward and backward: 4.96 ms
+// against 5.09 ms with chain_fwd (N 96, one round: 3.41 against 3.00 ms, and chain_fwd it is).
 //
-// Three compute waves hold the keys in registers (row layout of ChainRows; the P row slots of a lane are
+// Windowed over the staged 16-step chunks.  Three compute waves hold the keys (row layout of ChainRows; the P row
+// slots of a lane are
 // P-wide vectors, one per element, so the written row -- a wave-uniform slot -- is addressed with an
 // M0-relative move instead of a branch).  A fourth, producer wave stages the tokens of the next chunk in
 // LDS, and with one MFMA pass per chunk computes the chunk's Gram block E[s][u] = <k_s, q_u> and the
@@ -302,17 +296,10 @@ __device__ __forceinline__ u32 wavemax_key(u32 v) {
 // which the owner lane applies to its row's scores (rounded once per term, re-derived from the keys at
 // the next window).  The row norm of the written row is recomputed from its new elements.  The per-step
 // work left is the score, the argmax, and the one-row update.
-//
-// EM selects the key emission: CF_F32 the fp32 snapshots (kbuf); CF_BF the writer epilogue's bf16 copies with
-// kinv and valid; CF_NONE no key snapshots at all -- the row replay (rows_fwd with RF_CODES / RF_MEMQ) rebuilds
-// every key row bitwise from the address log and emits both copies, so the latency-bound chain carries no
-// snapshot bursts.
-#define FWD_THREADS (CHAIN_THREADS + 64)
-enum { CF_F32 = 0, CF_BF = 1, CF_NONE = 2 };
-template <int D, int P, typename TI, int EM>
-__global__ __attribute__((amdgpu_flat_work_group_size(FWD_THREADS, FWD_THREADS), amdgpu_waves_per_eu(2)))
-void chain_fwd(ChainFwdArgs a) {
-    constexpr bool MB = EM == CF_BF;
+#define REG_THREADS (CHAIN_THREADS + 64)
+template <int D, int P, typename TI>
+__global__ __attribute__((amdgpu_flat_work_group_size(REG_THREADS, REG_THREADS), amdgpu_waves_per_eu(2)))
+void chain_fwd_reg(ChainFwdArgs a) {
     constexpr int EPL = D / 16;
     constexpr int DP = D + 4;                           // padded LDS row: 16 rows at stride DP hit 16 bank groups
     constexpr int EPU = 16 / (int)sizeof(TI);          // token elements per uint4
@@ -427,13 +414,9 @@ void chain_fwd(ChainFwdArgs a) {
     const ChainRows<P> R(tid);
     const size_t sstride = (size_t)H * N * D;
     const size_t snap0 = ((size_t)b * a.NB + ts / G) * H + h;           // (b, ts / G, h): snapshot of block ts / G
-    float* kb = EM == CF_F32 ? a.kbuf + snap0 * N * D + (a.skip0 ? sstride : 0) : nullptr;   // skip0: the first slab is written
-    bf16_t* kbm = MB ? a.kbm + snap0 * N * D : nullptr;
-    float* kinvm = MB ? a.kinvm + snap0 * N : nullptr;
-    uint8_t* validm = MB ? a.validm + snap0 * N : nullptr;
+    float* kb = a.kbuf + snap0 * N * D + (a.skip0 ? sstride : 0);   // skip0: the first slab is written
     rowv Kv[EPL];                                       // Kv[e][j]: element e of this lane's slice of row j
     float o_me = 0.f, kinv_me;
-    bool vld_me;                                        // |K_me|^2 > 1e-12 (the epilogue's `valid`)
     {
         // the P rows' loads go out together (from row min(n, N - 1), unconditionally) and rows past N are
         // zeroed afterwards: a load per row behind a branch, used right away, waited for each row in turn
@@ -474,7 +457,6 @@ void chain_fwd(ChainFwdArgs a) {
             nsq0 = (c >> RS<P>::SH) == j ? sj : nsq0;
         }
         kinv_me = rsq_clamped(nsq0);
-        vld_me = nsq0 > 1e-12f;
         if (a.o0 && R.n_me < N) o_me = a.o0[(size_t)bh * N + R.n_me];
     }
     auto row_of = [&](int j, float* row) {
@@ -571,33 +553,17 @@ void chain_fwd(ChainFwdArgs a) {
             uint4 r[CHAIN_WAVES];
 #pragma unroll
             for (int w = 0; w < CHAIN_WAVES; w++) r[w] = s_red[par][w];
-            if (EM != CF_NONE && gc == 0 && (MB || t != ts || !a.skip0)) {   // the PRE-write key state of block t / G:
+            if (gc == 0 && (t != ts || !a.skip0)) {   // the PRE-write key state of block t / G:
                 u32 ro = roff;                              // every row group stores whole rows
                 int nvv = nvalid;
                 asm volatile("" : "+v"(ro), "+v"(nvv));     // per-snapshot offsets, not 16 live registers
-                if constexpr (MB) {                         // the writer epilogue: bf16 copy, kinv, valid
 #pragma unroll
-                    for (int jr = 0; jr < P; jr++) {
-                        float row[EPL];
-                        row_of(jr, row);
-                        if (jr < nvv) st_slice_bf_at<EPL>(kbm, (ro >> 1) + (u32)(jr * D * 2), row);
-                    }
-                    if (R.prim && valid_me) {
-                        kinvm[R.n_me] = kinv_me;
-                        validm[R.n_me] = vld_me ? 1 : 0;
-                    }
-                    kbm += sstride;
-                    kinvm += (size_t)H * N;
-                    validm += (size_t)H * N;
-                } else {
-#pragma unroll
-                    for (int jr = 0; jr < P; jr++) {
-                        float row[EPL];
-                        row_of(jr, row);
-                        if (jr < nvv) st_slice_at<EPL, true>(kb, ro + (u32)(jr * D * 4), row);
-                    }
-                    kb += sstride;
+                for (int jr = 0; jr < P; jr++) {
+                    float row[EPL];
+                    row_of(jr, row);
+                    if (jr < nvv) st_slice_at<EPL, true>(kb, ro + (u32)(jr * D * 4), row);
                 }
+                kb += sstride;
             }
             if (++gc == G) gc = 0;
             // waves in order = rows in order: strict '>' keeps the lowest row on ties
@@ -642,7 +608,6 @@ void chain_fwd(ChainFwdArgs a) {
                     if (a.oold && R.prim) a.oold[ix] = o_me;
                     o_me = omw * o_me + g;
                     kinv_me = rsq_clamped(kk);
-                    vld_me = kk > 1e-12f;
                     // all 16 entries: those at or before step j are never read again in this window
 #pragma unroll
                     for (int q4 = 0; q4 < CT / 4; q4++)
@@ -662,22 +627,434 @@ void chain_fwd(ChainFwdArgs a) {
     if (valid_me && R.prim) a.ofin[(size_t)bh * N + R.n_me] = o_me;
 }
 
+// ========================================================================================== chain_fwd
+// The sequential key chain: one workgroup per chain, the addresses decided by ONE wave over LDS records.
+//
+// A chain is a serial run of T dependent steps, so its time is the latency of a step, not bytes or flops.  With the
+// rows spread over three waves and the keys in registers (chain_fwd_reg) a step took 2,900 cycles, most of them in
+// the waves' meeting (LDS exchange and barrier) and in the owner's M0-relative register update.  Here:
+//   - wave 0 decides every step alone.  A lane scores rows NR lane .. NR lane + NR - 1 from the window's scores, a
+//     DPP maximum and NR ballots give the lowest competing row, and that row's record is read from LDS, blended
+//     with the token, written back, and its norm formed -- no barrier inside a 16-step window, no global access
+//     (a store would wait behind the CU's own snapshot stream) and no branch but the rare one below;
+//   - a record holds a row's key, its 16 scores of the window, and its occupancy, so a write reads and updates all
+//     of it with one address: lanes 0-15 take the scores (x <- (1 - g) x + g E[t][u], <(1-g) K + g k, q> by
+//     linearity), the others the occupancy (x <- (1 - g) x + g), in one fma;
+//   - waves 1-3 prepare the next window while it runs: tokens, the Gram block E and the scores of ALL rows, fp32
+//     MFMAs on the keys in LDS.  Rows that wave 0 writes meanwhile get scores from a key that may be half
+//     written; wave 0 computes those rows' scores again at the window's end (one 16-row tile gathered at the
+//     window's addresses, rows written twice twice) before anyone uses them;
+//   - the rows that compete (occupied ones, the lowest free one) are scalar masks, recomputed only when a write
+//     takes a row's occupancy across eps;
+//   - the cosines for the backward take the place of the used scores, and waves 1-3 store them behind the window.
+// Scores, norms, blends and the order of their sums are those of chain_fwd_reg: the two give the same bits.
+//
+// Measured per step (N 192, D 128, bf16; 48 or 252 chains alike): 0.42 us (about 1,000 cycles, 150 instructions of
+// one wave) against 1.22-1.36 us before, and 13 us a launch for the state's way into LDS and back.  B 8, T 1,024
+// as a stream of codes: 1,303 -> 538 us a call; B 256, T 256, N 96 forward and backward: 2,835 -> 2,431 us.
+template <int D, typename TI> struct ChainLds {
+    // a slot row's record (floats): the key, the window's 16 scores <K_n, q_u>, the occupancy, 3 pad; 16 rows'
+    // 16-byte reads at this stride start on 16 bank groups
+    static constexpr int DP = D + CT + 4;
+    static constexpr int DQ = D + 16 / (int)sizeof(TI);  // padded token row (elements), 16-byte rows
+    static constexpr int ES = CT + 4;                    // a step's row of E: 16 products, then its gate
+    // bytes of dynamic LDS for NP rows (N rounded up to 16)
+    static constexpr size_t bytes(int NP) {
+        return ((size_t)(NP + 1) * DP + NP + 2 * CT * ES + 2 * 4 * CT + 2 * CT) * 4 + 4 * CT * DQ * sizeof(TI);
+    }
+};
+constexpr int FWD_THREADS = 256;
+
+// row-sized vectors at 4-byte aligned addresses (gfx950 takes dword-aligned vector accesses)
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x3u __attribute__((ext_vector_type(3), aligned(4)));
+
+template <int D, int NR, typename TI, bool LOG>
+__global__ __attribute__((amdgpu_flat_work_group_size(FWD_THREADS, FWD_THREADS), amdgpu_waves_per_eu(1)))
+void chain_fwd(ChainFwdArgs a) {
+    typedef ChainLds<D, TI> Z;
+    typedef u32 u32x4v __attribute__((ext_vector_type(4)));
+    constexpr int EPL = D / 16, DP = Z::DP, DQ = Z::DQ, ES = Z::ES, SO = D;          // SO: the scores in a record
+    constexpr int KL = D / 4;                           // MFMA operand dims per lane group
+    constexpr int EPU = 16 / (int)sizeof(TI);           // token elements per 16 bytes
+    constexpr int RU = D / EPU;                         // 16-byte pieces per token row
+    constexpr int NU = 2 * CT * RU;                     // pieces per window: (q row, k row) per token
+    constexpr int HT = FWD_THREADS - 64;                // helper lanes
+    constexpr int UPT = (NU + HT - 1) / HT;
+    constexpr int TPW = (4 * NR + 2) / 3;               // row tiles per helper wave
+    const int T = a.T, H = a.H, N = a.N, ts = a.ts, te = a.te;
+    const int NP = (N + 15) & ~15;
+    extern __shared__ __align__(16) unsigned char smem[];
+    float* const s_tab = reinterpret_cast<float*>(smem);         // [NP + 1][DP] records; the last: lanes without a row
+    TI* const s_tk = reinterpret_cast<TI*>(s_tab + (NP + 1) * DP);     // [2][2][CT][DQ] tokens: q, k
+    float* const s_E = reinterpret_cast<float*>(s_tk + 4 * CT * DQ);   // [2][CT][ES] g_s <k_s, q_u>; g_s
+    float* const s_sc = s_E + 2 * CT * ES;                       // [2][CT][4] gate, 1 - gate, fr, 1 / |q|
+    float* const s_ki = s_sc + 2 * 4 * CT;                       // [NP] 1 / |K_n| (start)
+    float* const s_log = s_ki + NP;                              // [2][CT] the window's rows, their old occupancy
+    const int bh = blockIdx.x, b = bh / H, h = bh - b * H;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = tid & 15;
+    const int m16 = lane & 15, ag = lane >> 4;
+    const TI* __restrict__ qp = (const TI*)a.q;
+    const TI* __restrict__ kp = (const TI*)a.k;
+    const size_t tok0 = (size_t)b * T * H + h;
+    const int nwin = (te - ts + CT - 1) / CT;
+
+    u32x4v rq[UPT];
+    float rsv = 0.f;
+    const float* const gate_p = a.gate;
+    const float* const fr_p = a.frt ? a.fr : a.gate;
+    const int ht = tid - 64;
+    // helper lanes: window w's tokens and step scalars.  Loads go out unconditionally from clamped addresses;
+    // tokens past te are staged as 0 with gate 0, so a step past te changes nothing.
+    auto load_win = [&](int w) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < UPT; m++) {
+            const int u = min(ht + HT * m, NU - 1);
+            const int j = u / (2 * RU), arr = (u / RU) & 1, x = u % RU;
+            const int t = min(ts + w * CT + j, te - 1);
+            rq[m] = reinterpret_cast<const u32x4v*>((arr ? kp : qp) + (tok0 + (size_t)t * H) * D)[x];
+        }
+        const int t = min(ts + w * CT + (lane & (CT - 1)), te - 1);
+        const float* sp = lane < CT ? gate_p : fr_p;
+        rsv = sp[tok0 + (size_t)t * H];
+    };
+    auto store_win = [&](int w) __attribute__((always_inline)) {
+        const int pr = w & 1, left = te - ts - w * CT;
+#pragma unroll
+        for (int m = 0; m < UPT; m++) {
+            const int u = ht + HT * m;
+            const int j = u / (2 * RU), arr = (u / RU) & 1, x = u % RU;
+            if (u < NU) *reinterpret_cast<u32x4v*>(s_tk + ((pr * 2 + arr) * CT + j) * DQ + x * EPU) = j < left ? rq[m] : u32x4v{0, 0, 0, 0};
+        }
+        if (wave == 3 && lane < 2 * CT) {
+            const int j = lane & (CT - 1);
+            const float x = j < left ? rsv : 0.f;
+            float* sc = s_sc + (pr * CT + j) * 4;
+            if (lane < CT) { sc[0] = x; sc[1] = 1.f - x; s_E[(pr * CT + j) * ES + CT] = x; }
+            else sc[2] = a.frt ? x : a.fr[0];
+        }
+    };
+    // E[s][u] = g_s <k_s, q_u> and 1 / max(|q_u|, 1e-6) of window w, by one wave
+    auto gram = [&](int w) __attribute__((always_inline)) {
+        const int pr = w & 1;
+        const TI* tq = s_tk + (pr * 2 + 0) * CT * DQ;
+        const TI* tk = s_tk + (pr * 2 + 1) * CT * DQ;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i4 = 0; i4 < KL / 4; i4++) {
+            const float4 ka = ld4(tk + m16 * DQ + ag * KL + 4 * i4);
+            const float4 qb = ld4(tq + m16 * DQ + ag * KL + 4 * i4);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.x, qb.x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.y, qb.y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.z, qb.z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.w, qb.w, acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) s_E[(pr * CT + 4 * ag + r) * ES + m16] = s_sc[(pr * CT + 4 * ag + r) * 4] * acc[r];
+        const int u = lane >> 2, p4 = lane & 3;
+        float qq = 0.f;
+#pragma unroll
+        for (int i4 = 0; i4 < D / 16; i4++) {
+            const float4 x = ld4(tq + u * DQ + p4 * (D / 4) + 4 * i4);
+            qq = fmaf(x.x, x.x, qq); qq = fmaf(x.y, x.y, qq); qq = fmaf(x.z, x.z, qq); qq = fmaf(x.w, x.w, qq);
+        }
+        qq += dppf<SLOT_DPP_XOR1>(qq);
+        qq += dppf<SLOT_DPP_XOR2>(qq);
+        if (p4 == 0) s_sc[(pr * CT + u) * 4 + 3] = rsq_clamped(qq);
+    };
+    // the scores of 16 key rows (row: this lane's, one per m16) with window w's queries: lane (m16, ag) gets
+    // <K_row, q_u>, u = 4 ag .. 4 ag + 3
+    auto tile = [&](int w, int row) __attribute__((always_inline)) {
+        const TI* tq = s_tk + ((w & 1) * 2 + 0) * CT * DQ;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i4 = 0; i4 < KL / 4; i4++) {
+            const float4 qa = ld4(tq + m16 * DQ + ag * KL + 4 * i4);
+            const float4 kb = ld4(s_tab + row * DP + ag * KL + 4 * i4);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.x, kb.x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.y, kb.y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.z, kb.z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.w, kb.w, acc, 0, 0, 0);
+        }
+        return acc;
+    };
+    auto put_tile = [&](f32x4 acc, int row) __attribute__((always_inline)) {
+        *reinterpret_cast<f32x4*>(s_tab + row * DP + SO + 4 * ag) = acc;
+    };
+
+    // ---- start: the keys, the first two windows' tokens
+    if (wave > 0) load_win(0);
+    {
+        // every row's loads go out together, from row min(n, N - 1); rows past N are zeroed
+        const float* k0r = a.k0 ? a.k0 + (size_t)bh * N * D : nullptr;
+        const int rg = tid >> 4;
+#pragma unroll
+        for (int i0 = 0; i0 < 4 * NR; i0 += 4) {
+            float row[4][EPL];
+            if (k0r) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) ld_slice<EPL>(row[i], k0r + (size_t)min(rg + 16 * (i0 + i), N - 1) * D, c);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int n = rg + 16 * (i0 + i);
+                if (n < NP) {
+#pragma unroll
+                    for (int e = 0; e < EPL; e++) row[i][e] = k0r && n < N ? row[i][e] : 0.f;
+                    st_slice<EPL>(s_tab + n * DP, row[i], c);
+                    // each row's norm in the row update's order, so that a launch starts from bitwise the norm the
+                    // previous one ended with
+                    float kk = 0.f;
+#pragma unroll
+                    for (int e = 0; e < EPL; e++) kk = fmaf(row[i][e], row[i][e], kk);
+                    kk = rowsum16(kk);
+                    if (c == 0) s_ki[n] = rsq_clamped(kk);
+                }
+            }
+        }
+        if (tid < NP) s_tab[tid * DP + SO + CT] = a.o0 && tid < N ? a.o0[(size_t)bh * N + tid] : 0.f;
+    }
+    if (wave > 0) { store_win(0); load_win(1); }
+    __syncthreads();
+    for (int tau = wave; tau < NP / 16; tau += 4) put_tile(tile(0, 16 * tau + m16), 16 * tau + m16);
+    if (wave == 3) gram(0);
+    if (wave > 0) { store_win(1); load_win(2); }
+    __syncthreads();
+
+    if (wave > 0) {                                     // helpers
+        for (int w = 0; w < nwin; w++) {
+            f32x4 acc[TPW], lg[TPW];
+            float lw = 0.f;
+            const bool more = w + 1 < nwin;
+            if (more) {
+#pragma unroll
+                for (int i = 0; i < TPW; i++) {
+                    const int tau = wave - 1 + 3 * i;
+                    if (tau < NP / 16) acc[i] = tile(w + 1, 16 * tau + m16);
+                }
+                if (wave == 3) gram(w + 1);
+            }
+            __syncthreads();
+            // the window's cosines, which the chain left where the scores were, then the next window's scores there
+#pragma unroll
+            for (int i = 0; i < TPW; i++) {
+                const int tau = wave - 1 + 3 * i;
+                if (tau < NP / 16) {
+                    if (LOG) lg[i] = *reinterpret_cast<const f32x4*>(s_tab + (16 * tau + m16) * DP + SO + 4 * ag);
+                    if (more) put_tile(acc[i], 16 * tau + m16);
+                }
+            }
+            if (wave == 3) lw = s_log[lane & (2 * CT - 1)];
+            if (more) store_win(w + 2);
+            __syncthreads();
+            // loads before stores: the wait for a load covers every older operation
+            if (more) load_win(w + 3);
+            const int t0 = ts + w * CT;
+            if (LOG) {
+#pragma unroll
+                for (int i = 0; i < TPW; i++) {
+                    const int n = 16 * (wave - 1 + 3 * i) + m16;
+                    float* cl = a.cslog + ((size_t)bh * T + t0 + 4 * ag) * N + n;
+#pragma unroll
+                    for (int x = 0; x < 4; x++)
+                        if (n < N && t0 + 4 * ag + x < te) __builtin_nontemporal_store(lg[i][x], cl + (size_t)x * N);
+                }
+            }
+            if (wave == 3 && t0 + (lane & (CT - 1)) < te) {
+                const size_t ix = tok0 + (size_t)(t0 + (lane & (CT - 1))) * H;
+                if (lane < CT) a.am[ix] = __float_as_int(lw);
+                else if (LOG && lane < 2 * CT) a.oold[ix] = lw;
+            }
+        }
+    } else {
+        float ki[NR], oc[NR];                           // 1 / |K|, the occupancy term of the score
+        u64 tk[NR], el[NR];                             // occupied rows; rows that compete
+        int sofs[NR];
+        const float temp = a.temp[0];
+        const float eps = a.eps;
+        const bool occb = a.occb != 0;
+        // this lane's rows: n0 .. n0 + NR - 1 (one vector store per step logs their cosines)
+        const int n0 = NR * lane;
+        // the rows that compete: occupied ones and the lowest free one
+        auto compete = [&]() __attribute__((always_inline)) {
+            u32 first = ~0u;
+            u64 fm[NR];
+#pragma unroll
+            for (int r = 0; r < NR; r++) {
+                const int nl = (N - r + NR - 1) / NR;    // lanes whose row r exists
+                const u64 in = nl >= 64 ? ~0ull : ((1ull << max(nl, 0)) - 1ull);
+                fm[r] = in & ~tk[r];
+                el[r] = tk[r] & in;
+                if (fm[r]) first = min(first, (u32)(NR * __builtin_ctzll(fm[r]) + r));
+            }
+#pragma unroll
+            for (int r = 0; r < NR; r++)
+                if (fm[r] && first == (u32)(NR * __builtin_ctzll(fm[r]) + r)) el[r] |= fm[r] & (0ull - fm[r]);
+        };
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const int n = min(n0 + r, NP - 1);
+            sofs[r] = min(n0 + r, NP) * DP + SO;
+            ki[r] = s_ki[n];
+            const float o = s_tab[n * DP + SO + CT];
+            tk[r] = __ballot(o >= eps);
+            oc[r] = occb ? (o >= eps ? 1.f : 0.f) : o;
+        }
+        compete();
+        for (int w = 0; w < nwin; w++) {
+            const int t0 = ts + w * CT;
+            const TI* tkp = s_tk + ((w & 1) * 2 + 1) * CT * DQ;
+            // lanes 0-15 take a row's 16 scores through a step, lanes 16-63 its occupancy: x <- (1 - g) x + (g E or g)
+            const float* Ew = s_E + (w & 1) * CT * ES + min(lane, CT);
+            const float* sc = s_sc + (w & 1) * 4 * CT;
+            int amw = 0;                                // lanes j, j + 16, ..: the row that step j wrote
+            float oow = 0.f;                            // and its occupancy before
+            const int nst = min(CT, te - t0);
+            float Sc[NR];                               // the step's column of the scores
+#pragma unroll
+            for (int r = 0; r < NR; r++) Sc[r] = s_tab[sofs[r]];
+            // the step's scalars, key token and row of E, read a step ahead
+            float4 sv = ld4(sc);
+            float kv[EPL];
+            ld_slice<EPL>(kv, tkp, c);
+            float e1 = Ew[0];
+            auto step = [&](int j, int jn) __attribute__((always_inline)) {      // jn: the next step (j at the window's end)
+                const float g = sv.x, omw = sv.y, frv = sv.z, qi = sv.w;
+                int key[NR];
+                float cs[NR];                            // cosines of this lane's rows with the query
+                int m = (int)0x80000000;
+#pragma unroll
+                for (int r = 0; r < NR; r++) {
+                    cs[r] = (Sc[r] * ki[r]) * qi;
+                    const float z = fmaf(temp, cs[r], -(oc[r] * frv));
+                    const int zi = __float_as_int(z + 0.0f);
+                    const int zk = zi ^ ((zi >> 31) & 0x7fffffff);       // signed order = IEEE order
+                    key[r] = __builtin_amdgcn_inverse_ballot_w64(el[r]) ? zk : (int)0x80000000;
+                    m = max(m, key[r]);
+                }
+                m = max(m, (int)dppu<SLOT_DPP_XOR1>((u32)m));
+                m = max(m, (int)dppu<SLOT_DPP_XOR2>((u32)m));
+                m = max(m, (int)dppu<SLOT_DPP_HMIR>((u32)m));
+                m = max(m, (int)dppu<SLOT_DPP_MIR>((u32)m));
+                // row_bcast15 into rows 1 and 3, row_bcast31 into rows 2 and 3: lane 63 ends with the wave's maximum
+                m = max(m, __builtin_amdgcn_update_dpp((int)0x80000000, m, 0x142, 0xa, 0xf, false));
+                m = max(m, __builtin_amdgcn_update_dpp((int)0x80000000, m, 0x143, 0xc, 0xf, false));
+                m = __builtin_amdgcn_readlane(m, 63);
+                // the lowest competing row at the maximum (s_ff1 of 0 is -1: no row of this kind)
+                u32 row_u = ~0u;
+#pragma unroll
+                for (int r = 0; r < NR; r++) {
+                    const u64 eq = __ballot(key[r] == m) & el[r];
+                    u32 f;
+                    asm("s_ff1_i32_b64 %0, %1" : "=s"(f) : "s"(eq));
+                    row_u = min(row_u, f * NR + r);
+                }
+                const int am = (int)min((u32)__builtin_amdgcn_readfirstlane((int)row_u), (u32)(N - 1));
+                float old[EPL];
+                float* const rec = s_tab + am * DP;
+                ld_slice<EPL>(old, rec, c);
+                if (LOG) {                               // the step's cosines, in place of its scores
+#pragma unroll
+                    for (int r = 0; r < NR; r++) s_tab[sofs[r] + j] = cs[r];
+                }
+                float* const sr = rec + SO + min(lane, CT);
+                const float so = *sr;
+                asm volatile("" : : : "memory");         // the next step's reads go out behind this step's
+                float kn_[EPL], Sn[NR];
+                ld_slice<EPL>(kn_, tkp + jn * DQ, c);
+                const float en = Ew[jn * ES];
+                const float4 svn = ld4(sc + 4 * jn);
+#pragma unroll
+                for (int r = 0; r < NR; r++) Sn[r] = s_tab[sofs[r] + jn];
+                asm volatile("" : : : "memory");
+                amw = c == j ? am : amw;
+                // the row's scores with the window's later queries (its earlier entries hold cosines); its occupancy
+                const float sn = lane > j ? fmaf(omw, so, e1) : so;
+                *sr = sn;
+                float nv[EPL], part = 0.f;
+#pragma unroll
+                for (int e = 0; e < EPL; e++) nv[e] = blend(old[e], kv[e], g, omw);
+                st_slice<EPL>(rec, nv, c);               // (the four row groups hold and store the same values)
+#pragma unroll
+                for (int e = 0; e < EPL; e++) part = fmaf(nv[e], nv[e], part);
+                if (LOG) {
+                    const float oo = readlanef(so, CT);
+                    oow = c == j ? oo : oow;
+                }
+                const float kn = rsq_clamped(rowsum16(part));
+                const float s1 = readlanef(sn, jn);
+#pragma unroll
+                for (int r = 0; r < NR; r++) {
+                    const bool me = n0 + r == am;
+                    ki[r] = me ? kn : ki[r];
+                    Sc[r] = me ? s1 : Sn[r];
+                }
+                sv = svn;
+                e1 = en;
+#pragma unroll
+                for (int e = 0; e < EPL; e++) kv[e] = kn_[e];
+                // the row's occupancy crossed eps (its first write), or the scores take the occupancy itself
+                const u32 cross = (u32)(__ballot(sn >= eps) ^ __ballot(so >= eps));
+                if (__builtin_expect((cross & (1u << CT)) || !occb, 0)) {
+                    const float on = readlanef(sn, CT);
+                    const bool now = on >= eps;
+                    const int al = am / NR, ar = am - NR * al;
+#pragma unroll
+                    for (int r = 0; r < NR; r++) {
+                        const u64 bit = ar == r ? 1ull << al : 0ull;
+                        tk[r] = now ? tk[r] | bit : tk[r] & ~bit;
+                        oc[r] = n0 + r == am ? (occb ? (now ? 1.f : 0.f) : on) : oc[r];
+                    }
+                    compete();
+                }
+            };
+            // four steps a turn: constant offsets inside it, and code that stays a small part of the instruction
+            // cache (all 16 unrolled, a short call spent its time fetching them)
+#pragma unroll 1
+            for (int j0 = 0; j0 < nst; j0 += 4) {
+                step(j0, j0 + 1);
+                step(j0 + 1, j0 + 2);
+                step(j0 + 2, j0 + 3);
+                step(j0 + 3, min(j0 + 4, CT - 1));
+            }
+            if (lane < CT) {
+                s_log[lane] = __int_as_float(amw);
+                if (LOG) s_log[CT + lane] = oow;
+            }
+            __syncthreads();
+            const bool more = w + 1 < nwin;
+            f32x4 acc;
+            if (more) acc = tile(w + 1, amw);            // the written rows' scores, from their new keys
+            __syncthreads();
+            if (more) put_tile(acc, amw);
+            wave_lds_sync();
+        }
+        for (int r = 0; r < NR; r++)
+            if (n0 + r < N) a.ofin[(size_t)bh * N + n0 + r] = s_tab[(n0 + r) * DP + SO + CT];
+    }
+    for (int n = tid >> 4; n < N; n += FWD_THREADS / 16) {
+        float row[EPL];
+        ld_slice<EPL>(row, s_tab + n * DP, c);
+        st_slice<EPL>(a.kfin + ((size_t)bh * N + n) * D, row, c);
+    }
+}
+
 // =========================================================================================== rows_fwd
 struct RowsFwdArgs {
-    const void* v; const float* gate; const int32_t* am; const float* v0;
-    float* vbuf; float* vold; float* vfin;
+    const void* k; const void* v; const float* gate; const int32_t* am;
+    const float* k0; const float* v0;                    // start state (NULL: zero), end state (kfin may be NULL)
+    float* kfin; float* vfin;
+    float* kold; float* vold;                            // undo log (NULL: not differentiated)
     int T, H, N, G, NB;
     int ts, te;                                          // steps [ts, te); ts % G == 0
-    bf16_t* vbm;                                         // the writer-epilogue emission (NULL: fp32 vbuf)
-    int v0bs, vfbs, skip0;                               // as ChainFwdArgs' k0bs, kfbs, skip0
-    // RF_CODES / RF_MEMQ: the key replay (tokens k, start state k0 (B*H, N, D) or NULL, end state kfin) and the
-    // emission of both copies -- integer codes + per-group scales (RF_CODES), or the quantiser's values (bits
-    // 0: the plain values) as bf16 with kinv and valid of the emitted keys (RF_MEMQ, into kbm, vbm, kinvm,
-    // validm)
-    const void* k; const float* k0; float* kfin;
-    int bits, group;
-    bf16_t* kbm; float* kinvm; uint8_t* validm;
-    int8_t* kcode; float* kscale; int8_t* vcode; float* vscale;
+    // chain (b, h) of a start state is slab b * k0bs + h (v0bs), of an end state b * kfbs + h (vfbs): H for
+    // (B*H, N, D) buffers; NB * H where a chunk of the pipeline starts from (ends in) the fp32 snapshot of its
+    // first (next) block.  skip0: that first snapshot is already written, by the previous chunk.
+    int k0bs, kfbs, v0bs, vfbs, skip0;
+    float* kbuf; float* vbuf;                            // RF_F32: fp32 snapshots
+    bf16_t* kbm; bf16_t* vbm; float* kinvm; uint8_t* validm;         // RF_MEM: bf16 copies, kinv and valid
+    int8_t* kcode; float* kscale; int8_t* vcode; float* vscale;      // RF_CODES: integer codes, group scales
+    int bits, group;                                     // the storage quantiser (RF_MEM: bits 0 = plain values)
 };
 
 // The storage quantiser _fq (memlm_sh.py:221-228) over a row slice held the row-group way: EPL / 4 pieces of
@@ -737,24 +1114,23 @@ __device__ __forceinline__ u32 pack_codes4(const float* cd) {
            (((u32)(int)cd[3] & 0xffu) << 24);
 }
 
-// 512 lanes = 32 rows of one chain per workgroup; grid (B*H, ceil(N/32)).  Replays every row's value from
-// the address log and emits the value snapshots with full-row non-temporal stores.  A row changes only at
+// 512 lanes = 32 rows of one chain per workgroup; grid (B*H, ceil(N/32)).  Replays every row's key and value
+// from the address log and emits both snapshots with full-row non-temporal stores.  A row changes only at
 // its own writes, so the replay visits events, not steps: per 16-step piece of the staged address log a
 // lane forms the mask of steps that wrote its row (4 LDS reads) and, with the piece's G-aligned snapshot
 // steps, walks the set bits in step order (snapshot first: it is the PRE-write state).
-// EM: RF_F32 fp32 value snapshots; RF_BF bf16 value copies; RF_CODES / RF_MEMQ also replay the KEY rows (the
-// chain's own blend on the same staged token values, so bitwise the chain's keys) and emit both copies in
-// the storage quantiser's integer form (RF_CODES) or as the writer epilogue's bf16 values with kinv and
-// valid (RF_MEMQ).  The key state crosses the forward pipeline's inner chunk boundaries through kfin (each
-// chunk's replay ends by writing it and the next starts from it), apart from the chain's own carry.
-enum { RF_F32 = 0, RF_BF = 1, RF_CODES = 2, RF_MEMQ = 3 };
+// The key replay is the chain's own blend on the same token values, so bitwise the chain's keys.
+// EM: RF_F32 fp32 snapshots (RF_F32V: of the values alone, where the chain writes the keys'); RF_CODES the storage
+// quantiser's integer form; RF_MEM the writer epilogue's bf16 copies with kinv and valid, after the quantiser
+// where bits > 0.  The states cross the forward pipeline's inner chunk boundaries through kfin and vfin (each
+// chunk's replay ends by writing them and the next starts from them), apart from the chain's own carry.
+enum { RF_F32 = 0, RF_CODES = 1, RF_MEM = 2, RF_F32V = 3 };
 template <int D, typename TI, int EM>
 ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
     constexpr int EPL = D / 16;
     constexpr int NP = EPL / 4;
-    constexpr bool MB = EM == RF_BF;
-    constexpr bool KR = EM >= RF_CODES;                  // the key rows are replayed too
-    constexpr int TC = 256;                              // staged steps: 2 KB of LDS, so the replay blocks fit beside two chain blocks on a CU
+    constexpr bool KR = EM != RF_F32V;                   // the key rows too
+    constexpr int TC = 256;                              // staged steps: 2 KB of LDS, so the replay blocks fit beside a chain block on a CU
     __shared__ __align__(16) int s_am[TC];
     __shared__ float s_g[TC];
     const int T = a.T, H = a.H, N = a.N, G = a.G;
@@ -769,33 +1145,29 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
 #pragma unroll
     for (int e = 0; e < EPL; e++) { V[e] = 0.f; K[e] = 0.f; }
     if (live && a.v0) ld_slice<EPL>(V, a.v0 + ((size_t)(b * a.v0bs + h) * N + n) * D, c);
-    if (KR && live && a.k0) ld_slice<EPL>(K, a.k0 + ((size_t)bh * N + n) * D, c);
-    const size_t vrow0 = (((size_t)b * a.NB + a.ts / G) * H + h) * N * D + (size_t)(live ? n : 0) * D;
-    float* vb = EM == RF_F32 ? a.vbuf + vrow0 : nullptr;
-    bf16_t* vbh = MB ? a.vbm + vrow0 : nullptr;
-    const size_t sstride = (size_t)H * N * D;
-    // RF_CODES / RF_MEMQ outputs: the row's snapshot index advances by one (b, nb, h) slab per snapshot
+    if (KR && live && a.k0) ld_slice<EPL>(K, a.k0 + ((size_t)(b * a.k0bs + h) * N + n) * D, c);
+    const size_t sstride = (size_t)H * N;
+    // the row's snapshot index, advanced by one (b, nb, h) slab per snapshot
     size_t srow = (((size_t)b * a.NB + a.ts / G) * H + h) * N + (size_t)(live ? n : 0);
-    const int gpr = KR && EM == RF_CODES ? D / a.group : 0;   // scales per row
-    auto emit = [&]() {
+    const int gpr = EM == RF_CODES ? D / a.group : 0;     // scales per row
+    // What the row emits changes only with the row: it is formed at the first snapshot after a write (`fresh`
+    // false) and held for the later ones, packed as stored.  A block of G steps writes at most G of the N rows,
+    // and the quantiser's IEEE divisions had been most of the kernel's issue.
+    bool fresh = false;
+    u32x2 kx[NP], vx[NP];                                // codes (x) or bf16 values of each piece
+    float ks[NP], vs[NP];                                // scales; RF_MEM: ks[0] = |K|^2 of the emitted key
+    auto form = [&]() {
+        float kv[EPL], vv[EPL];
         if constexpr (EM == RF_CODES) {
-            float kv[EPL], kc[EPL], ks[NP], vv[EPL], vc[EPL], vs[NP];
+            float kc[EPL], vc[EPL];
             fq_slice<EPL>(K, a.bits, a.group, kv, kc, ks);
             fq_slice<EPL>(V, a.bits, a.group, vv, vc, vs);
-            int8_t* kcr = a.kcode + srow * D;
-            int8_t* vcr = a.vcode + srow * D;
 #pragma unroll
             for (int jj = 0; jj < NP; jj++) {
-                __builtin_nontemporal_store(pack_codes4(kc + 4 * jj), reinterpret_cast<u32*>(kcr + 64 * jj + 4 * c));
-                __builtin_nontemporal_store(pack_codes4(vc + 4 * jj), reinterpret_cast<u32*>(vcr + 64 * jj + 4 * c));
-                const int ch = 64 * jj + 4 * c;          // the group's first lane stores its scale
-                if (ch % a.group == 0) {
-                    a.kscale[srow * gpr + ch / a.group] = ks[jj];
-                    a.vscale[srow * gpr + ch / a.group] = vs[jj];
-                }
+                kx[jj].x = pack_codes4(kc + 4 * jj);
+                vx[jj].x = pack_codes4(vc + 4 * jj);
             }
-        } else if constexpr (EM == RF_MEMQ) {
-            float kv[EPL], vv[EPL];
+        } else {
             if (a.bits) {
                 float cd[EPL], sc[NP];
                 fq_slice<EPL>(K, a.bits, a.group, kv, cd, sc);
@@ -807,12 +1179,39 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
             float sq = 0.f;
 #pragma unroll
             for (int e = 0; e < EPL; e++) sq = fmaf(kv[e], kv[e], sq);
-            const float nsq = rowsum16(sq);
-            st_slice_bf_at<EPL>(a.kbm + srow * D, 8u * (u32)c, kv);
-            st_slice_bf_at<EPL>(a.vbm + srow * D, 8u * (u32)c, vv);
+            ks[0] = rowsum16(sq);
+#pragma unroll
+            for (int jj = 0; jj < NP; jj++) {
+                kx[jj] = u32x2{pack_bf16x2(kv[4 * jj], kv[4 * jj + 1]), pack_bf16x2(kv[4 * jj + 2], kv[4 * jj + 3])};
+                vx[jj] = u32x2{pack_bf16x2(vv[4 * jj], vv[4 * jj + 1]), pack_bf16x2(vv[4 * jj + 2], vv[4 * jj + 3])};
+            }
+        }
+    };
+    auto emit = [&]() {
+        if constexpr (EM == RF_CODES) {
+            int8_t* kcr = a.kcode + srow * D;
+            int8_t* vcr = a.vcode + srow * D;
+#pragma unroll
+            for (int jj = 0; jj < NP; jj++) {
+                const int ch = 64 * jj + 4 * c;
+                __builtin_nontemporal_store(kx[jj].x, reinterpret_cast<u32*>(kcr + ch));
+                __builtin_nontemporal_store(vx[jj].x, reinterpret_cast<u32*>(vcr + ch));
+                if (ch % a.group == 0) {                 // the group's first lane stores its scale
+                    a.kscale[srow * gpr + ch / a.group] = ks[jj];
+                    a.vscale[srow * gpr + ch / a.group] = vs[jj];
+                }
+            }
+        } else {
+            char* kr = reinterpret_cast<char*>(a.kbm + srow * D) + 8 * c;
+            char* vr = reinterpret_cast<char*>(a.vbm + srow * D) + 8 * c;
+#pragma unroll
+            for (int jj = 0; jj < NP; jj++) {
+                __builtin_nontemporal_store(kx[jj], reinterpret_cast<u32x2*>(kr + 128 * jj));
+                __builtin_nontemporal_store(vx[jj], reinterpret_cast<u32x2*>(vr + 128 * jj));
+            }
             if (c == 0) {                                // kinv and valid of the emitted (quantised) keys
-                a.kinvm[srow] = rsqrtf(fmaxf(nsq, 1e-12f));
-                a.validm[srow] = nsq > 1e-12f ? 1 : 0;
+                a.kinvm[srow] = rsqrtf(fmaxf(ks[0], 1e-12f));
+                a.validm[srow] = ks[0] > 1e-12f ? 1 : 0;
             }
         }
     };
@@ -843,35 +1242,38 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
                 const int i = __builtin_ctz(ev);
                 ev &= ev - 1;
                 if ((sm >> i) & 1u) {
-                    if constexpr (MB) { st_slice_bf_at<EPL>(vbh, 8u * (u32)c, V); vbh += sstride; }
-                    else if constexpr (EM == RF_F32) {
-                        if (t0 + j0 + i != a.ts || !a.skip0) st_slice_nt<EPL>(vb, V, c);   // skip0: already written
-                        vb += sstride;
+                    if constexpr (EM == RF_F32 || EM == RF_F32V) {
+                        if (t0 + j0 + i != a.ts || !a.skip0) {               // skip0: already written
+                            if (KR) st_slice_nt<EPL>(a.kbuf + srow * D, K, c);
+                            st_slice_nt<EPL>(a.vbuf + srow * D, V, c);
+                        }
                     } else {
+                        if (!fresh) { form(); fresh = true; }
                         emit();
-                        srow += (size_t)H * N;
                     }
+                    srow += sstride;
                 }
                 if ((hm >> i) & 1u) {
                     const size_t ix = tok0 + (size_t)(t0 + j0 + i) * H;
                     const float g = s_g[j0 + i], omw = 1.f - g;
-                    float vv[EPL];
+                    float vv[EPL], kk[EPL];
                     ld_slice<EPL>(vv, vp + ix * D, c);
-                    if (a.vold) st_slice_nt<EPL>(a.vold + ix * D, V, c);      // streaming, as kold
+                    if (KR) ld_slice<EPL>(kk, kp + ix * D, c);
+                    if (a.vold) {                        // the undo log, read only by the backward: streaming stores
+                        if (KR) st_slice_nt<EPL>(a.kold + ix * D, K, c);
+                        st_slice_nt<EPL>(a.vold + ix * D, V, c);
+                    }
 #pragma unroll
                     for (int e = 0; e < EPL; e++) V[e] = blend(V[e], vv[e], g, omw);
-                    if constexpr (KR) {
-                        float kk[EPL];
-                        ld_slice<EPL>(kk, kp + ix * D, c);
 #pragma unroll
-                        for (int e = 0; e < EPL; e++) K[e] = blend(K[e], kk[e], g, omw);
-                    }
+                    for (int e = 0; e < EPL; e++) K[e] = KR ? blend(K[e], kk[e], g, omw) : 0.f;
+                    fresh = false;
                 }
             }
         }
     }
     if (live) st_slice<EPL>(a.vfin + ((size_t)(b * a.vfbs + h) * N + n) * D, V, c);
-    if (KR && live && a.kfin) st_slice<EPL>(a.kfin + ((size_t)bh * N + n) * D, K, c);   // the key carry (inner chunks)
+    if (KR && live && a.kfin) st_slice<EPL>(a.kfin + ((size_t)(b * a.kfbs + h) * N + n) * D, K, c);   // the key carry (inner chunks)
 }
 
 // =========================================================================================== rows_bwd
@@ -914,7 +1316,6 @@ __device__ __forceinline__ void ldg_untracked(u32x4& d, const void* p) {
 __device__ __forceinline__ void ldg_untracked(float& d, const void* p) {
     asm volatile("global_load_dword %0, %1, off" : "+v"(d) : "v"(p));
 }
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void ldg_untracked_nt(u32x2& d, const void* p) {
     asm volatile("global_load_dwordx2 %0, %1, off nt" : "+v"(d) : "v"(p));
 }
@@ -2309,14 +2710,20 @@ __global__ __launch_bounds__(256) void reduce_parts(const float* __restrict__ pa
 
 // ===================================================================================== host dispatch
 template <int D, typename TI>
-hipError_t launch_chain_fwd(const ChainFwdArgs& a, int B, hipStream_t st) {
-    dim3 grid(B * a.H), block(FWD_THREADS);
-#define SLOT_CF(PP) if (a.N <= 4 * CHAIN_WAVES * PP) { \
-        if (a.kbm) slothost::launch((chain_fwd<D, PP, TI, CF_BF>), grid, block, 0, st, a); \
-        else if (a.kbuf) slothost::launch((chain_fwd<D, PP, TI, CF_F32>), grid, block, 0, st, a); \
-        else slothost::launch((chain_fwd<D, PP, TI, CF_NONE>), grid, block, 0, st, a); \
+hipError_t launch_chain_fwd(const ChainFwdArgs& a, int B, bool reg, hipStream_t st) {
+    if constexpr (D == 128) {
+        if (reg) {
+            slothost::launch((chain_fwd_reg<D, 16, TI>), dim3(B * a.H), dim3(REG_THREADS), 0, st, a);
+            return hipGetLastError();
+        }
+    }
+    const dim3 grid(B * a.H), block(FWD_THREADS);
+    const uint32_t lds = (uint32_t)ChainLds<D, TI>::bytes((a.N + 15) & ~15);
+#define SLOT_CF(RR) if (a.N <= 64 * RR) { \
+        if (a.cslog) slothost::launch((chain_fwd<D, RR, TI, true>), grid, block, lds, st, a); \
+        else slothost::launch((chain_fwd<D, RR, TI, false>), grid, block, lds, st, a); \
         return hipGetLastError(); }
-    SLOT_CF(1) SLOT_CF(2) SLOT_CF(4) SLOT_CF(8) SLOT_CF(16)
+    SLOT_CF(1) SLOT_CF(2) SLOT_CF(3)
 #undef SLOT_CF
     return hipErrorInvalidValue;
 }
@@ -2482,17 +2889,17 @@ static int check_common(int64_t B, int64_t T, int64_t H, int64_t N, int64_t D, i
 }
 
 // What one forward call emits.  FE_F32: fp32 snapshots (kbuf, vbuf).  FE_MEM: the writer epilogue's bf16
-// copies with kinv and valid, the keys from the chain (kbm, vbm, kinvm, validm).  FE_MEMQ: the same outputs
-// with the storage quantiser applied (bits > 0; bits 0 = plain values), both copies from the row replay.
-// FE_CODES: the quantiser's integer codes and per-group scales of both copies, from the row replay.
-enum { FE_F32 = 0, FE_MEM = 1, FE_MEMQ = 2, FE_CODES = 3 };
+// copies with kinv and valid, after the storage quantiser where bits > 0.  FE_CODES: the quantiser's integer
+// codes and per-group scales of both copies.
+enum { FE_F32 = 0, FE_MEM = 1, FE_CODES = 2 };
 struct FwdOut {
     int mode;
     float* kbuf; float* vbuf;
     bf16_t* kbm; bf16_t* vbm; float* kinvm; uint8_t* validm;
     int8_t* kcode; float* kscale; int8_t* vcode; float* vscale;
     int bits, group;
-    float* kcarry;                                       // FE_MEMQ / FE_CODES: the key replay's chunk carry
+    float* kcarry;                                       // FE_MEM / FE_CODES: the key replay's chunk carry
+    bool one;                                            // no carry to hand: one chunk
 };
 
 // chunk length of the forward pipeline (a multiple of G); T < 512 runs as one chunk
@@ -2558,15 +2965,14 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
                     float* kfin, float* vfin, float* ofin, void* stream) {
     if (int r = check_common(B, T, H, N, D, G, dtype)) return r;
     const int mode = o.mode;
-    const bool kr = mode == FE_MEMQ || mode == FE_CODES;         // the row replay emits the keys
-    int64_t cb[FWD_MAX_CHUNKS + 1];
-    const int nch = fwd_chunks(B, T, H, N, G, cb);
+    int64_t cb[FWD_MAX_CHUNKS + 1] = {0, T};
+        const int nch = o.one ? 1 : fwd_chunks(B, T, H, N, G, cb);
     if (!k || !q || !v || !gate || !fr || !temp || !am || !kfin || !vfin || !ofin ||
         (mode == FE_F32 && (!o.kbuf || !o.vbuf)) ||
-        ((mode == FE_MEM || mode == FE_MEMQ) && (!o.kbm || !o.vbm || !o.kinvm || !o.validm)) ||
-        (mode == FE_CODES && (!o.kcode || !o.kscale || !o.vcode || !o.vscale)) || (kr && nch > 1 && !o.kcarry))
+        (mode == FE_MEM && (!o.kbm || !o.vbm || !o.kinvm || !o.validm)) ||
+        (mode == FE_CODES && (!o.kcode || !o.kscale || !o.vcode || !o.vscale)) || (mode != FE_F32 && nch > 1 && !o.kcarry))
         return fail(SLOTSCAN_ERR_NULL, "slotscan_fwd: a required pointer is NULL");
-    if (kr)
+    if (mode != FE_F32)
         if (int r = check_q(o.bits, o.group, D, mode == FE_CODES)) return r;
     if ((kold == nullptr) != (oold == nullptr) || (kold == nullptr) != (vold == nullptr) ||
         (kold == nullptr) != (cslog == nullptr))
@@ -2578,26 +2984,27 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
     hipStream_t st = (hipStream_t)stream;
     const int NB = (int)((T + G - 1) / G);
     const bool f32 = mode == FE_F32;
-    ChainFwdArgs ca{q, k, gate, fr, temp, k0, o0, f32 ? o.kbuf : nullptr, am, kold, oold, cslog, kfin, ofin,
-                    (int)T, (int)H, (int)N, (int)G, NB, eps, fr_per_token ? 1 : 0, occ_bin ? 1 : 0, 0, (int)T,
-                    mode == FE_MEM ? o.kbm : nullptr, o.kinvm, o.validm, (int)H, (int)H, 0};
-    RowsFwdArgs ra{v, gate, am, v0, f32 ? o.vbuf : nullptr, vold, vfin, (int)T, (int)H, (int)N, (int)G, NB, 0,
-                   (int)T, o.vbm, (int)H, (int)H, 0,
-                   k, k0, nullptr, o.bits, o.group, o.kbm, o.kinvm, o.validm, o.kcode, o.kscale, o.vcode, o.vscale};
+    // the register-resident chain: built for D = 128 and more than 96 rows, where chain_fwd's records leave room for
+    // one workgroup on each of the 256 CUs
+    const bool reg = f32 && nch > 1 && D == 128 && N > 96 && B * H > 256;
+    ChainFwdArgs ca{q, k, gate, fr, temp, k0, o0, am, oold, cslog, kfin, ofin, (int)T, (int)H, (int)N, eps,
+                    fr_per_token ? 1 : 0, occ_bin ? 1 : 0, 0, (int)T, o.kbuf, kold, (int)G, NB, (int)H, (int)H, 0};
+    RowsFwdArgs ra{k, v, gate, am, k0, v0, nullptr, vfin, kold, vold, (int)T, (int)H, (int)N, (int)G, NB, 0, (int)T,
+                   (int)H, (int)H, (int)H, (int)H, 0, o.kbuf, o.vbuf, o.kbm, o.vbm, o.kinvm, o.validm,
+                   o.kcode, o.kscale, o.vcode, o.vscale, o.bits, o.group};
     // Long sequences run as a two-stream pipeline over step chunks of a multiple of G: the key chain of
     // chunk c + 1 (latency-bound, caller's stream) overlaps the row replay of chunk c (HBM-bound, the
     // library's side stream); the last chunk's replay has no chain to overlap and runs on the caller's stream
-    // behind its chain, after the side stream's replays.  fp32 contract: the state crosses an inner chunk boundary te as the snapshot
-    // of block te / G, which is exactly the state there -- a chunk ends by writing it (it is its next block's
-    // PRE-write snapshot) and the next chunk starts from it without storing it again.  The other contracts
-    // emit no fp32 state, so the chain carries its keys in kfin, the value replay its values in vfin, and a
-    // key replay its keys in kcarry (the chain may already be overwriting kfin while the replay of an
-    // earlier chunk runs).  The occupancy crosses through ofin; the last chunk writes kfin, vfin, ofin.
+    // behind its chain, after the side stream's replays.  The chain carries its keys from chunk to chunk in kfin
+    // and its occupancy in ofin.  The replay carries both states (its keys apart from the chain's, which may
+    // already be overwriting kfin while the replay of an earlier chunk runs): with fp32 snapshots through the
+    // snapshot of the next block, te / G, which is exactly the state there -- a chunk ends by writing it and
+    // the next starts from it without storing it again -- else through kcarry and vfin.
     hipStream_t side = nullptr;
     hipEvent_t* ev = nullptr;
     if (nch > 1)
         if (int r = slothost::side_stream(&side, &ev, nch + 1)) return r;
-    dim3 grid((unsigned)(B * H), (unsigned)((N + 31) / 32)), block(512);
+    const dim3 grid((unsigned)(B * H), (unsigned)((N + 31) / 32)), block(512);
     hipError_t e;
     for (int c = 0; c < nch; c++) {
         ca.ts = ra.ts = (int)cb[c];
@@ -2605,27 +3012,34 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
         const bool inner_end = ca.te < T;
         if (c > 0) {
             ca.o0 = ofin;
-            if (!f32) {
-                ca.k0 = kfin;
-                ra.v0 = vfin;
-                if (kr) ra.k0 = o.kcarry;
-            } else {                                     // from the snapshot slab of block ts / G
-                ca.k0 = o.kbuf + (size_t)(ca.ts / G) * H * N * D;
+            ca.k0 = reg ? o.kbuf + (size_t)(ca.ts / G) * H * N * D : kfin;
+            if (f32) {
+                ca.k0bs = NB * (int)H;
+                ca.skip0 = 1;
+                ra.k0 = o.kbuf + (size_t)(ra.ts / G) * H * N * D;
                 ra.v0 = o.vbuf + (size_t)(ra.ts / G) * H * N * D;
-                ca.k0bs = ra.v0bs = NB * (int)H;
-                ca.skip0 = ra.skip0 = 1;
+                ra.k0bs = ra.v0bs = NB * (int)H;
+                ra.skip0 = 1;
+            } else {
+                ra.k0 = o.kcarry;
+                ra.v0 = vfin;
             }
         }
-        if (kr) ra.kfin = inner_end ? o.kcarry : nullptr;
-        if (f32) {                                       // an inner chunk ends in the next block's slab
-            ca.kfin = inner_end ? o.kbuf + (size_t)(ca.te / G) * H * N * D : kfin;
+        if (f32) {
+            ra.kfin = inner_end ? o.kbuf + (size_t)(ra.te / G) * H * N * D : nullptr;
             ra.vfin = inner_end ? o.vbuf + (size_t)(ra.te / G) * H * N * D : vfin;
-            ca.kfbs = ra.vfbs = inner_end ? NB * (int)H : (int)H;
+            ra.kfbs = ra.vfbs = inner_end ? NB * (int)H : (int)H;
+            if (reg) {                                   // the chain writes and carries the keys' snapshots itself
+                ca.kfin = inner_end ? ra.kfin : kfin;
+                ca.kfbs = ra.kfbs;
+            }
+        } else {
+            ra.kfin = inner_end ? o.kcarry : nullptr;
         }
         {
             slothost::Scope sc(SLOTSCAN_K_CHAIN_FWD, st);
-            if (D == 128) e = dtype == SLOTSCAN_BF16 ? launch_chain_fwd<128, bf16_t>(ca, (int)B, st) : launch_chain_fwd<128, float>(ca, (int)B, st);
-            else e = dtype == SLOTSCAN_BF16 ? launch_chain_fwd<64, bf16_t>(ca, (int)B, st) : launch_chain_fwd<64, float>(ca, (int)B, st);
+            if (D == 128) e = dtype == SLOTSCAN_BF16 ? launch_chain_fwd<128, bf16_t>(ca, (int)B, reg, st) : launch_chain_fwd<128, float>(ca, (int)B, reg, st);
+            else e = dtype == SLOTSCAN_BF16 ? launch_chain_fwd<64, bf16_t>(ca, (int)B, reg, st) : launch_chain_fwd<64, float>(ca, (int)B, reg, st);
         }
         if (e != hipSuccess) return hip_fail(e, "chain_fwd launch");
         hipStream_t rs = st;
@@ -2641,9 +3055,9 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
         }
         {
             slothost::Scope sc(SLOTSCAN_K_ROWS_FWD, rs);
-#define SLOT_RF(DD, TT) { if (mode == FE_MEM) slothost::launch((rows_fwd<DD, TT, RF_BF>), grid, block, 0, rs, ra); \
-                          else if (mode == FE_MEMQ) slothost::launch((rows_fwd<DD, TT, RF_MEMQ>), grid, block, 0, rs, ra); \
+#define SLOT_RF(DD, TT) { if (mode == FE_MEM) slothost::launch((rows_fwd<DD, TT, RF_MEM>), grid, block, 0, rs, ra); \
                           else if (mode == FE_CODES) slothost::launch((rows_fwd<DD, TT, RF_CODES>), grid, block, 0, rs, ra); \
+                          else if (reg) slothost::launch((rows_fwd<DD, TT, RF_F32V>), grid, block, 0, rs, ra); \
                           else slothost::launch((rows_fwd<DD, TT, RF_F32>), grid, block, 0, rs, ra); }
             if (D == 128) {
                 if (dtype == SLOTSCAN_BF16) SLOT_RF(128, bf16_t) else SLOT_RF(128, float)
@@ -2682,6 +3096,7 @@ extern "C" int slotscan_fwd_mem(const void* k, const void* q, const void* v, int
                                 float* kfin, float* vfin, float* ofin, void* stream) {
     FwdOut o{};
     o.mode = FE_MEM; o.kbm = (bf16_t*)kb; o.vbm = (bf16_t*)vb; o.kinvm = kinv; o.validm = valid;
+    o.one = true;
     return scan_fwd(k, q, v, dtype, gate, fr, fr_per_token, temp, B, T, H, N, D, G, eps, occ_bin, k0, v0, o0,
                     o, am, kold, vold, oold, cslog, kfin, vfin, ofin, stream);
 }
@@ -2700,7 +3115,7 @@ extern "C" int slotscan_fwd_memq(const void* k, const void* q, const void* v, in
                                  float* kold, float* vold, float* oold, float* cslog,
                                  float* kfin, float* vfin, float* ofin, float* kcarry, void* stream) {
     FwdOut o{};
-    o.mode = FE_MEMQ; o.kbm = (bf16_t*)kb; o.vbm = (bf16_t*)vb; o.kinvm = kinv; o.validm = valid;
+    o.mode = FE_MEM; o.kbm = (bf16_t*)kb; o.vbm = (bf16_t*)vb; o.kinvm = kinv; o.validm = valid;
     o.bits = bits; o.group = (int)group; o.kcarry = kcarry;
     return scan_fwd(k, q, v, dtype, gate, fr, fr_per_token, temp, B, T, H, N, D, G, eps, occ_bin, k0, v0, o0,
                     o, am, kold, vold, oold, cslog, kfin, vfin, ofin, stream);

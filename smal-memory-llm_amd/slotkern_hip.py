@@ -98,8 +98,8 @@ def _carry(B, T, H, N, D, G, dev):
 def _fwd(k_, q_, v_, g, fr_, frt, temp_, N, G, eps, occ_bin, dt, logs, state=None, mem=False, bits=0, group=16):
     """One forward launch.  mem=False: returns (kbuf, vbuf, am, logs..., final state).  mem=True: the writer
     epilogue is fused in, and the first two results are replaced by the four (kb, vb, kinv, valid); with
-    bits > 0 it is the quantised epilogue (slotscan_fwd_memq: the storage quantiser's values, kinv and valid
-    of the quantised keys)."""
+    bits > 0 after the storage quantiser (kinv and valid of the quantised keys); both run slotscan_fwd_memq, whose
+    key carry lets a long scan run as the chunk pipeline."""
     B, T, H, D = k_.shape
     NB = (T + G - 1) // G
     dev = k_.device
@@ -121,17 +121,13 @@ def _fwd(k_, q_, v_, g, fr_, frt, temp_, N, G, eps, occ_bin, dt, logs, state=Non
     head = pre + (L.ptr(k0), L.ptr(v0), L.ptr(o0))
     tail = (L.ptr(am), L.ptr(kold), L.ptr(vold), L.ptr(oold), L.ptr(cslog), L.ptr(kfin), L.ptr(vfin),
             L.ptr(ofin))
-    if mem and bits:
+    if mem:
         kc = _carry(B, T, H, N, D, G, dev)
         rc = L.lib().slotscan_fwd_memq(*pre, int(bits), int(group), L.ptr(k0), L.ptr(v0), L.ptr(o0), L.ptr(kbuf),
                                        L.ptr(vbuf), L.ptr(kinv), L.ptr(valid), *tail, L.ptr(kc), L.stream_of(dev))
         L.check(rc, "slotscan_fwd_memq")
         return (kbuf, vbuf, kinv, valid), am, kold, vold, oold, cslog, kfin, vfin, ofin
     tail = tail + (L.stream_of(dev),)
-    if mem:
-        rc = L.lib().slotscan_fwd_mem(*head, L.ptr(kbuf), L.ptr(vbuf), L.ptr(kinv), L.ptr(valid), *tail)
-        L.check(rc, "slotscan_fwd_mem")
-        return (kbuf, vbuf, kinv, valid), am, kold, vold, oold, cslog, kfin, vfin, ofin
     rc = L.lib().slotscan_fwd(*head, L.ptr(kbuf), L.ptr(vbuf), *tail)
     L.check(rc, "slotscan_fwd")
     return kbuf, vbuf, am, kold, vold, oold, cslog, kfin, vfin, ofin
