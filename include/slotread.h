@@ -47,6 +47,18 @@ int slotread_bwd(const void* q, const void* kbuf, const void* vbuf, const float*
                  int64_t D, int64_t G, void* dq, void* dkbuf, void* dvbuf, float* dkinv, float* dscale,
                  void* stream);
 
+/* The read's query preparation in one pass (memlm_sh.py:379-393): qn = q / max(|q|, 1e-6) with the norm rounded to
+ * bf16, scale = exp(log_rsel) exp(sharp tanh(s / sharp)) (sharp 0: exp(s); s NULL: exp(log_rsel)).
+ *   q, qn (rows, D) bf16, 16-byte aligned, D 64 or 128;  s, scale (rows) fp32;  log_rsel one fp32.
+ * Backward: dqn (rows, D) bf16 and dscale (rows) fp32 in; dq (rows, D) bf16, ds (rows, with s), dlog_rsel (one) out;
+ * workspace slotread_prep_workspace(rows, D) bytes. */
+size_t slotread_prep_workspace(int64_t rows, int64_t D);
+int slotread_prep_fwd(const void* q, const float* s, const float* log_rsel, float sharp, int64_t rows, int64_t D,
+                      void* qn, float* scale, void* stream);
+int slotread_prep_bwd(const void* q, const float* s, const float* scale, const void* dqn, const float* dscale,
+                      float sharp, int64_t rows, int64_t D, void* workspace, void* dq, float* ds, float* dlog_rsel,
+                      void* stream);
+
 #ifdef __cplusplus
 }
 #endif

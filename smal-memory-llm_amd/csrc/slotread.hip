@@ -1079,6 +1079,125 @@ __global__ __launch_bounds__(READ_THREADS) __attribute__((amdgpu_waves_per_eu(AC
     }
 }
 
+// ============================================================================================ query preparation
+// qn = q / max(|q|, 1e-6) in bf16 and the multiplier exp(log_rsel) exp(C tanh(s / C)) of every read query, in one pass.
+// D / 8 lanes hold a query (16 bytes each), 256 lanes a workgroup: bound by its bytes (q in, qn out).  As torch
+// operations the same took seven passes and eleven launches forward and about fifteen backward; B 64, T 1024, H 6,
+// NQ 2, D 128, a reader layer's forward and backward: 4,390 us with them, 3,033 us with these.
+struct PrepArgs {
+    const bf16_t* q; const float* s; const float* log_rsel;
+    const bf16_t* dqn; const float* dscale;              // backward: upstream gradients
+    bf16_t* qn;                                          // forward: unit queries; backward: dq
+    float* scale;                                        // forward: written; backward: read
+    float* ds; float* part;                              // backward: part: one sum of dscale * scale per workgroup
+    int64_t rows; float sharp;                           // sharp: C, or 0 for exp(s)
+};
+constexpr int PREP_THREADS = 256;
+
+template <int L> __device__ __forceinline__ float prep_sum(float v) {       // over L = 8 or 16 consecutive lanes
+    v += dppf<SLOT_DPP_XOR1>(v);
+    v += dppf<SLOT_DPP_XOR2>(v);
+    v += dppf<SLOT_DPP_HMIR>(v);
+    if constexpr (L == 16) v += dppf<SLOT_DPP_MIR>(v);
+    return v;
+}
+__device__ __forceinline__ void prep_unpack(uint4 r, float* x) {
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        x[2 * i] = __uint_as_float(w[i] << 16);
+        x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+}
+
+template <int D>
+__global__ __launch_bounds__(PREP_THREADS) void read_prep(PrepArgs a) {
+    constexpr int L = D / 8, RW = PREP_THREADS / L;      // lanes per query, queries per workgroup
+    const int tid = threadIdx.x;
+    const int64_t row0 = (int64_t)blockIdx.x * RW, row = row0 + tid / L;
+    if (row < a.rows) {
+        const int64_t at = row * D + 8 * (tid % L);
+        float x[8], qq = 0.f;
+        prep_unpack(*reinterpret_cast<const uint4*>(a.q + at), x);
+#pragma unroll
+        for (int e = 0; e < 8; e++) qq = fmaf(x[e], x[e], qq);
+        // the norm is rounded to bf16 before the division, as in q's dtype
+        const float nb = bf16_round(fmaxf(__fsqrt_rn(prep_sum<L>(qq)), 1e-6f));
+        uint4 r;
+        r.x = pack_bf16x2(x[0] / nb, x[1] / nb);
+        r.y = pack_bf16x2(x[2] / nb, x[3] / nb);
+        r.z = pack_bf16x2(x[4] / nb, x[5] / nb);
+        r.w = pack_bf16x2(x[6] / nb, x[7] / nb);
+        *reinterpret_cast<uint4*>(a.qn + at) = r;
+    }
+    if (tid < RW && row0 + tid < a.rows) {
+        float m = expf(a.log_rsel[0]);
+        if (a.s) {
+            const float sv = a.s[row0 + tid];
+            m *= expf(a.sharp != 0.f ? a.sharp * tanhf(sv / a.sharp) : sv);
+        }
+        a.scale[row0 + tid] = m;
+    }
+}
+
+// dq = dqn / nb - q [|q| >= 1e-6] <dqn, q> / (nb^2 |q|) (the norm's rounding to bf16 passes the gradient), in fp32 and
+// rounded once; ds = dscale scale (1 - tanh^2); the workgroup's sum of dscale scale for log_rsel.
+template <int D>
+__global__ __launch_bounds__(PREP_THREADS) void read_prep_bwd(PrepArgs a) {
+    constexpr int L = D / 8, RW = PREP_THREADS / L;
+    const int tid = threadIdx.x;
+    const int64_t row0 = (int64_t)blockIdx.x * RW, row = row0 + tid / L;
+    if (row < a.rows) {
+        const int64_t at = row * D + 8 * (tid % L);
+        float x[8], d[8], qq = 0.f, dot = 0.f;
+        prep_unpack(*reinterpret_cast<const uint4*>(a.q + at), x);
+        prep_unpack(*reinterpret_cast<const uint4*>(a.dqn + at), d);
+#pragma unroll
+        for (int e = 0; e < 8; e++) { qq = fmaf(x[e], x[e], qq); dot = fmaf(x[e], d[e], dot); }
+        const float nrm = __fsqrt_rn(prep_sum<L>(qq));
+        dot = prep_sum<L>(dot);
+        const float nb = bf16_round(fmaxf(nrm, 1e-6f));
+        const float co = nrm >= 1e-6f ? dot / nb / nb / nrm : 0.f;
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) y[e] = d[e] / nb - co * x[e];
+        uint4 r;
+        r.x = pack_bf16x2(y[0], y[1]);
+        r.y = pack_bf16x2(y[2], y[3]);
+        r.z = pack_bf16x2(y[4], y[5]);
+        r.w = pack_bf16x2(y[6], y[7]);
+        *reinterpret_cast<uint4*>(a.qn + at) = r;
+    }
+    if (tid < 64) {                                      // (RW <= 32: one wave)
+        float t = 0.f;
+        if (tid < RW && row0 + tid < a.rows) {
+            t = a.dscale[row0 + tid] * a.scale[row0 + tid];
+            if (a.s) {
+                const float sv = a.s[row0 + tid];
+                const float th = a.sharp != 0.f ? tanhf(sv / a.sharp) : 0.f;
+                a.ds[row0 + tid] = t * (1.f - th * th);
+            }
+        }
+        t = wavesum(t);
+        if (tid == 0) a.part[blockIdx.x] = t;
+    }
+}
+
+// the workgroups' partials in a fixed order (1,024 lanes, then a tree)
+__global__ __launch_bounds__(1024) void read_prep_reduce(const float* __restrict__ part, int n, float* out) {
+    __shared__ float s_w[16];
+    float t = 0.f;
+    for (int i = threadIdx.x; i < n; i += 1024) t += part[i];
+    t = wavesum(t);
+    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float u = 0.f;
+        for (int i = 0; i < 16; i++) u += s_w[i];
+        out[0] = u;
+    }
+}
+
 }  // namespace
 
 // ======================================================================================== C-ABI
@@ -1193,4 +1312,47 @@ extern "C" int slotread_bwd(const void* q, const void* kbuf, const void* vbuf, c
     }
     if (e != hipSuccess) return hip_fail(e, "read_bwd launch");
     return 0;
+}
+
+static int check_prep(int64_t rows, int64_t D) {
+    if (rows < 1 || (D != 64 && D != 128)) return fail(SLOTSCAN_ERR_SHAPE, "slotread_prep: rows >= 1, D 64 or 128");
+    if (rows > 0x7fffffffLL * 16) return fail(SLOTSCAN_ERR_SHAPE, "slotread_prep: too many rows");
+    return 0;
+}
+
+extern "C" size_t slotread_prep_workspace(int64_t rows, int64_t D) {
+    if (rows < 1 || (D != 64 && D != 128)) return 0;
+    const int64_t rw = PREP_THREADS / (D / 8);
+    return (size_t)((rows + rw - 1) / rw) * sizeof(float);
+}
+
+extern "C" int slotread_prep_fwd(const void* q, const float* s, const float* log_rsel, float sharp, int64_t rows,
+                                 int64_t D, void* qn, float* scale, void* stream) {
+    if (int r = check_prep(rows, D)) return r;
+    if (!q || !log_rsel || !qn || !scale) return fail(SLOTSCAN_ERR_NULL, "slotread_prep_fwd: a required pointer is NULL");
+    if (!al16(q) || !al16(qn)) return fail(SLOTSCAN_ERR_ALIGN, "slotread_prep_fwd: q and qn must be 16-byte aligned");
+    PrepArgs a{(const bf16_t*)q, s, log_rsel, nullptr, nullptr, (bf16_t*)qn, scale, nullptr, nullptr, rows, sharp};
+    const dim3 grid((unsigned)(slotread_prep_workspace(rows, D) / sizeof(float)));
+    if (D == 128) slothost::launch(read_prep<128>, grid, dim3(PREP_THREADS), 0, (hipStream_t)stream, a);
+    else slothost::launch(read_prep<64>, grid, dim3(PREP_THREADS), 0, (hipStream_t)stream, a);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : hip_fail(e, "read_prep launch");
+}
+
+extern "C" int slotread_prep_bwd(const void* q, const float* s, const float* scale, const void* dqn,
+                                 const float* dscale, float sharp, int64_t rows, int64_t D, void* workspace, void* dq,
+                                 float* ds, float* dlog_rsel, void* stream) {
+    if (int r = check_prep(rows, D)) return r;
+    if (!q || !scale || !dqn || !dscale || !workspace || !dq || !dlog_rsel || (s && !ds))
+        return fail(SLOTSCAN_ERR_NULL, "slotread_prep_bwd: a required pointer is NULL");
+    if (!al16(q) || !al16(dqn) || !al16(dq))
+        return fail(SLOTSCAN_ERR_ALIGN, "slotread_prep_bwd: q, dqn and dq must be 16-byte aligned");
+    PrepArgs a{(const bf16_t*)q, s, nullptr, (const bf16_t*)dqn, dscale, (bf16_t*)dq, const_cast<float*>(scale), ds,
+               (float*)workspace, rows, sharp};
+    const int n = (int)(slotread_prep_workspace(rows, D) / sizeof(float));
+    if (D == 128) slothost::launch(read_prep_bwd<128>, dim3((unsigned)n), dim3(PREP_THREADS), 0, (hipStream_t)stream, a);
+    else slothost::launch(read_prep_bwd<64>, dim3((unsigned)n), dim3(PREP_THREADS), 0, (hipStream_t)stream, a);
+    slothost::launch(read_prep_reduce, dim3(1), dim3(1024), 0, (hipStream_t)stream, (const float*)workspace, n, dlog_rsel);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : hip_fail(e, "read_prep_bwd launch");
 }

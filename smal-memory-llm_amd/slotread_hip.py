@@ -93,18 +93,71 @@ def slot_read(q, kbuf, buf, kinv, valid, scale, G):
     return _SlotReadHip.apply(q, kbuf, buf, kinv, valid, scale, int(G))
 
 
-def shared_read(q, kbuf, buf, kinv, valid, log_rsel, G, s=None, rsharp=None):
-    """memlm_sh.py:379-397 given the projected read queries q (B,T,H,NQ,D): q / max(|q|, 1e-6) in q's dtype
-    (:379), multiplier exp(log_rsel) (:383) times exp(rsharp * tanh(s / rsharp)) when s (B,T,H,NQ) is given
-    (:385-393)."""
+def _al16(x):
+    """x contiguous at a 16-byte aligned address (a view may start anywhere in its storage)."""
+    x = x.contiguous()
+    return x.clone() if x.data_ptr() % 16 else x
+
+
+class _PrepHip(torch.autograd.Function):
+    """(qn, scale) of the projected queries q (B,T,H,NQ,D) bf16, s (B,T,H,NQ) fp32 or None, log_rsel (one value)."""
+
+    @staticmethod
+    def forward(ctx, q, s, log_rsel, sharp):
+        q_ = _al16(q)
+        s_ = None if s is None else s.contiguous()
+        D = q.shape[-1]
+        qn = torch.empty(q.shape, device=q.device, dtype=torch.bfloat16)
+        scale = torch.empty(q.shape[:-1], device=q.device, dtype=torch.float32)
+        rc = L.lib().slotread_prep_fwd(L.ptr(q_), L.ptr(s_), L.ptr(log_rsel.reshape(1)), sharp, scale.numel(), D,
+                                       L.ptr(qn), L.ptr(scale), L.stream_of(q.device))
+        L.check(rc, "slotread_prep_fwd")
+        ctx.save_for_backward(q_, s_, scale)
+        ctx.meta = (sharp, log_rsel.shape)
+        return qn, scale
+
+    @staticmethod
+    def backward(ctx, dqn, dscale):
+        q_, s_, scale = ctx.saved_tensors
+        sharp, lshape = ctx.meta
+        D, n, dev = q_.shape[-1], scale.numel(), q_.device
+        dqn, dscale = _al16(dqn.to(torch.bfloat16)), dscale.contiguous()
+        dq = torch.empty(q_.shape, device=dev, dtype=torch.bfloat16)
+        ds = None if s_ is None else torch.empty(s_.shape, device=dev, dtype=torch.float32)
+        dl = torch.empty(1, device=dev, dtype=torch.float32)
+        ws = torch.empty(L.lib().slotread_prep_workspace(n, D), device=dev, dtype=torch.uint8)
+        rc = L.lib().slotread_prep_bwd(L.ptr(q_), L.ptr(s_), L.ptr(scale), L.ptr(dqn), L.ptr(dscale), sharp, n, D,
+                                       L.ptr(ws), L.ptr(dq), L.ptr(ds), L.ptr(dl), L.stream_of(dev))
+        L.check(rc, "slotread_prep_bwd")
+        return dq, ds, dl.reshape(lshape), None
+
+
+def _prep(q, log_rsel, s, rsharp):
+    """(unit queries, multiplier) of memlm_sh.py:379-393.  bf16 queries with one log_rsel and an s of their own shape --
+    what the layer passes -- take one kernel each way (one pass over q instead of seven; measured there); other
+    dtypes, and a log_rsel or s that broadcasts, the same expressions in torch."""
+    B, T, H, NQ, D = q.shape
+    if (q.is_cuda and q.dtype == torch.bfloat16 and D in _SUPPORTED_D and q.numel() and torch.is_tensor(log_rsel)
+            and log_rsel.numel() == 1 and log_rsel.device == q.device and log_rsel.is_floating_point()
+            and (rsharp is None or isinstance(rsharp, (int, float)))
+            and (s is None or (s.shape == q.shape[:-1] and s.device == q.device and s.is_floating_point()))):
+        return _PrepHip.apply(q, None if s is None else s.float(), log_rsel.float(),
+                              0.0 if s is None or not rsharp else float(rsharp))
     qn = q / q.float().norm(dim=-1, keepdim=True).clamp_min(1e-6).to(q.dtype)
-    B, T, H, NQ, _ = q.shape
     scale = torch.exp(log_rsel.float()).expand(B, T, H, NQ)
     if s is not None:
         sf = s.float()
         if rsharp:
             sf = rsharp * torch.tanh(sf / rsharp)
         scale = scale * torch.exp(sf)
+    return qn, scale
+
+
+def shared_read(q, kbuf, buf, kinv, valid, log_rsel, G, s=None, rsharp=None):
+    """memlm_sh.py:379-397 given the projected read queries q (B,T,H,NQ,D): q / max(|q|, 1e-6) in q's dtype
+    (:379), multiplier exp(log_rsel) (:383) times exp(rsharp * tanh(s / rsharp)) when s (B,T,H,NQ) is given
+    (:385-393)."""
+    qn, scale = _prep(q, log_rsel, s, rsharp)
     return slot_read(qn, kbuf, buf, kinv, valid, scale, G)
 
 
@@ -204,12 +257,5 @@ def slot_read_out(q, kbuf, buf, kinv, valid, scale, G, wo, delta=None):
 def shared_read_out(q, kbuf, buf, kinv, valid, log_rsel, G, wo, s=None, rsharp=None, delta=None):
     """memlm_sh.py:379-397 then :499-501: shared_read's query preparation and multiplier, the read, and the
     wo_tk projection added to the window output delta, in one op."""
-    qn = q / q.float().norm(dim=-1, keepdim=True).clamp_min(1e-6).to(q.dtype)
-    B, T, H, NQ, _ = q.shape
-    scale = torch.exp(log_rsel.float()).expand(B, T, H, NQ)
-    if s is not None:
-        sf = s.float()
-        if rsharp:
-            sf = rsharp * torch.tanh(sf / rsharp)
-        scale = scale * torch.exp(sf)
+    qn, scale = _prep(q, log_rsel, s, rsharp)
     return slot_read_out(qn, kbuf, buf, kinv, valid, scale, G, wo, delta=delta)
