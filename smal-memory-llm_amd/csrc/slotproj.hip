@@ -261,6 +261,87 @@ __global__ __launch_bounds__(PTHREADS) void proj_gemm(ProjArgs p) {
     else epilogue(std::false_type{});
 }
 
+// ------------------------------------------------------------------------------------ few rows
+// The same product and epilogue for the row counts whose 256 x 256 tiles leave most of the chip idle (a block of
+// generated tokens, a short training batch).  It is bound by the latency of getting wo and rd to the MFMAs, so
+// the work is cut the other way: a workgroup owns 16 columns x 16 RM rows, its 8 waves split K (wave w takes the
+// 32-wide k steps w, w + 8, ..), and every operand goes straight from global memory into the MFMA layout --
+// lane l holds k 8 (l >> 4) .. + 7 of row l & 15 -- up to SU steps in flight and no LDS or barrier in the loop.  The
+// waves' fp32 partials meet in LDS and are summed in wave order.
+constexpr int SWAVES = 8, SU = 6;
+typedef float f32x4p __attribute__((ext_vector_type(4)));
+
+template <int RM>
+__global__ __launch_bounds__(64 * SWAVES) void proj_rows(ProjArgs p) {
+    constexpr int SR = 16 + 4;                             // padded partial row (floats)
+    __shared__ __align__(16) float s_p[SWAVES][16 * RM][SR];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, ag = lane >> 4;
+    const int n0 = 16 * blockIdx.x, m0 = 16 * RM * blockIdx.y;
+    const int KS = p.K / 32;
+    const bf16_t* gw = p.w + (size_t)(n0 + l16) * p.K + 8 * ag;
+    const bf16_t* ga[RM];
+#pragma unroll
+    for (int i = 0; i < RM; i++) ga[i] = p.a + (size_t)min(m0 + 16 * i + l16, p.M - 1) * p.K + 8 * ag;
+    f32x4p acc[RM];
+#pragma unroll
+    for (int i = 0; i < RM; i++) acc[i] = f32x4p{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wave; k0 < KS; k0 += SWAVES * SU) {
+        u32x4v w[SU], a[SU][RM];
+#pragma unroll
+        for (int u = 0; u < SU; u++) {                     // past the end: the last step again, not used
+            const int k = 32 * min(k0 + SWAVES * u, KS - 1);
+            w[u] = *reinterpret_cast<const u32x4v*>(gw + k);
+#pragma unroll
+            for (int i = 0; i < RM; i++) a[u][i] = *reinterpret_cast<const u32x4v*>(ga[i] + k);
+        }
+#pragma unroll
+        for (int u = 0; u < SU; u++)
+            if (k0 + SWAVES * u < KS) {
+#pragma unroll
+                for (int i = 0; i < RM; i++)
+                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[u]),
+                                                                     __builtin_bit_cast(bf16x8, a[u][i]), acc[i], 0, 0, 0);
+            }
+    }
+    // lane l, register r: column n0 + 4 (l >> 4) + r of row m0 + 16 i + (l & 15)
+#pragma unroll
+    for (int i = 0; i < RM; i++) *reinterpret_cast<f32x4p*>(&s_p[wave][16 * i + l16][4 * ag]) = acc[i];
+    __syncthreads();
+    for (int u = tid; u < 16 * RM * 4; u += 64 * SWAVES) {
+        const int r = u >> 2, c = 4 * (u & 3);
+        if (m0 + r >= p.M) continue;
+        f32x4p t = *reinterpret_cast<const f32x4p*>(&s_p[0][r][c]);
+#pragma unroll
+        for (int w = 1; w < SWAVES; w++) t += *reinterpret_cast<const f32x4p*>(&s_p[w][r][c]);
+        uint2 o = make_uint2(pack_bf16x2(t[0], t[1]), pack_bf16x2(t[2], t[3]));
+        const size_t at = (size_t)(m0 + r) * p.N + n0 + c;
+        if (p.d) {                                         // the bf16 Linear output, then the bf16 residual add
+            const float4 x = ld4(reinterpret_cast<const bf16_t*>(&o)), d = ld4(p.d + at);
+            o = make_uint2(pack_bf16x2(x.x + d.x, x.y + d.y), pack_bf16x2(x.z + d.z, x.w + d.w));
+        }
+        *reinterpret_cast<uint2*>(p.out + at) = o;
+    }
+}
+
+// out (M, N) = a w^T (+ d): proj_rows while its workgroups are at most two per CU, else proj_gemm.  Measured (us, proj_gemm
+// against proj_rows; N x K, rows): 2048 x 1536: 39 against 3.7 (1 row), 40 / 8.9 (64), 42 / 16 (256: 512 workgroups),
+// 42 / 32 (512), 43 / 66 (1,024); 512 x 512: 20 / 16 (1,024: 512), 20 / 31 (2,048); 2048 x 2048: 53 / 29 (256: 512),
+// 53 / 58 (512).
+constexpr int64_t ROWS_MAX_WG = 512;
+static hipError_t launch_proj(const ProjArgs& a, hipStream_t st) {
+    const unsigned nx = (unsigned)(a.N / 16);
+    if ((int64_t)nx * ((a.M + 63) / 64) <= ROWS_MAX_WG) {
+        const dim3 block(64 * SWAVES);
+        if (a.M <= 16) slothost::launch(proj_rows<1>, dim3(nx, 1), block, 0, st, a);
+        else if (a.M <= 32) slothost::launch(proj_rows<2>, dim3(nx, 1), block, 0, st, a);
+        else slothost::launch(proj_rows<4>, dim3(nx, (unsigned)((a.M + 63) / 64)), block, 0, st, a);
+    } else {
+        const int groups = (a.mblocks + PXCD - 1) / PXCD;
+        slothost::launch(proj_gemm, dim3((unsigned)(groups * PXCD * a.nblocks)), dim3(PTHREADS), 0, st, a);
+    }
+    return hipGetLastError();
+}
+
 // ------------------------------------------------------------------------------------ the backward's GEMMs
 // dWo = dDelta^T rd: C (N, K) = A^T B with A = dDelta (M, N) and B = rd (M, K), both token-major, the tokens
 // the reduction.  The same 256 x 256 tile, 4 waves and 4-stage ring of direct global -> LDS loads as
@@ -556,13 +637,12 @@ extern "C" int slotproj_fwd(const void* rd, const void* wo, const void* delta, i
         return fail(SLOTSCAN_ERR_ALIGN, "slotproj_fwd: rd, wo, delta and out must be 16-byte aligned");
     ProjArgs a{(const bf16_t*)rd, (const bf16_t*)wo, (const bf16_t*)delta, (bf16_t*)out, (int)M, (int)N, (int)K,
                (int)((M + PT - 1) / PT), (int)(N / PT)};
-    const int groups = (a.mblocks + PXCD - 1) / PXCD;
     hipStream_t st = (hipStream_t)stream;
+    hipError_t e;
     {
         slothost::Scope sc(SLOTSCAN_K_PROJ, st);
-        slothost::launch(proj_gemm, dim3((unsigned)(groups * PXCD * a.nblocks)), dim3(PTHREADS), 0, st, a);
+        e = launch_proj(a, st);
     }
-    hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "proj_gemm launch");
     return 0;
 }
