@@ -98,12 +98,13 @@ def check(rc, what):
 
 
 def ptr(t):
-    """Device pointer of a tensor, or None."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device pointer of a tensor (a plain int: the argtypes convert it), or None."""
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    # the raw handle of torch.cuda.current_stream(device), without building the Stream object (2 us a call)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def dtype_code(dt):
