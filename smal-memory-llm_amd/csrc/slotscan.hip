@@ -48,6 +48,7 @@ typedef uint32_t u32;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 #define SLOT_CT 16          // tokens per staged chunk
 #define CHAIN_WAVES 3
@@ -274,11 +275,11 @@ __device__ __forceinline__ u32 wavemax_key(u32 v) {
 }
 
 // The key chain with its keys in registers, which also writes the fp32 key snapshots.  It serves the fp32 contract
-// where the chains are more than one round of chain_fwd's workgroups (below) and the forward runs as the chunk
-// pipeline: the pipeline is then bound by its snapshot bytes, and this kernel, half of a CU's registers a
-// workgroup, holds every chain at once and writes the keys' half of them while it steps, in the first chunk
-// too, where the replay has nothing to do yet.  B 64, T 1024, H 6, N 192, D 128, forward and backward: 4.96 ms
-// against 5.09 ms with chain_fwd (N 96, one round: 3.41 against 3.00 ms, and chain_fwd it is).
+// where the chains are more than one round of chain_fwd's workgroups (below): the forward is then bound by its
+// snapshot bytes, and this kernel, half of a CU's registers a workgroup, holds twice the chains at once and writes
+// the keys' half of them while it steps, also where the replay has nothing to do yet.  H 6, N 192, D 128: B 64, T 1024
+// forward and backward 4.96 ms against 5.09 ms with chain_fwd; B 256, T 256 forward 2.29 against 2.77 ms; B 64, T 256
+// 0.67 against 0.77 ms (N 96, one round, B 64, T 1024: 3.41 against 3.00 ms, and chain_fwd it is).
 //
 // Windowed over the staged 16-step chunks.  Three compute waves hold the keys (row layout of ChainRows; the P row
 // slots of a lane are
@@ -1185,6 +1186,16 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
                 kx[jj] = u32x2{pack_bf16x2(kv[4 * jj], kv[4 * jj + 1]), pack_bf16x2(kv[4 * jj + 2], kv[4 * jj + 3])};
                 vx[jj] = u32x2{pack_bf16x2(vv[4 * jj], vv[4 * jj + 1]), pack_bf16x2(vv[4 * jj + 2], vv[4 * jj + 3])};
             }
+            if constexpr (NP == 2) {                     // lanes c, c ^ 1 trade pieces: the even one then holds 8
+                const bool odd = c & 1;                  // channels of the first half, the odd one of the second
+                auto trade = [&](u32x2* x) {
+                    const u32x2 snd = odd ? x[0] : x[1];
+                    const u32x2 rcv = {dppu<SLOT_DPP_XOR1>(snd.x), dppu<SLOT_DPP_XOR1>(snd.y)};
+                    if (odd) x[0] = rcv; else x[1] = rcv;
+                };
+                trade(kx);
+                trade(vx);
+            }
         }
     };
     auto emit = [&]() {
@@ -1202,12 +1213,15 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
                 }
             }
         } else {
-            char* kr = reinterpret_cast<char*>(a.kbm + srow * D) + 8 * c;
-            char* vr = reinterpret_cast<char*>(a.vbm + srow * D) + 8 * c;
-#pragma unroll
-            for (int jj = 0; jj < NP; jj++) {
-                __builtin_nontemporal_store(kx[jj], reinterpret_cast<u32x2*>(kr + 128 * jj));
-                __builtin_nontemporal_store(vx[jj], reinterpret_cast<u32x2*>(vr + 128 * jj));
+            const int o = NP == 2 ? (c & 1) * 128 + (c >> 1) * 16 : 8 * c;
+            char* kr = reinterpret_cast<char*>(a.kbm + srow * D) + o;
+            char* vr = reinterpret_cast<char*>(a.vbm + srow * D) + o;
+            if constexpr (NP == 2) {                     // 16 bytes a lane
+                __builtin_nontemporal_store(u32x4{kx[0].x, kx[0].y, kx[NP - 1].x, kx[NP - 1].y}, reinterpret_cast<u32x4*>(kr));
+                __builtin_nontemporal_store(u32x4{vx[0].x, vx[0].y, vx[NP - 1].x, vx[NP - 1].y}, reinterpret_cast<u32x4*>(vr));
+            } else {
+                __builtin_nontemporal_store(kx[0], reinterpret_cast<u32x2*>(kr));
+                __builtin_nontemporal_store(vx[0], reinterpret_cast<u32x2*>(vr));
             }
             if (c == 0) {                                // kinv and valid of the emitted (quantised) keys
                 a.kinvm[srow] = rsqrtf(fmaxf(ks[0], 1e-12f));
@@ -1306,7 +1320,6 @@ struct RowsBwdArgs {
 // explicit vmcnt whose asm operands are the destinations, so no use can be scheduled before the wait; "+v"
 // keeps each destination in place, so no copy of a value that has not arrived can be made.  Used where the
 // compiler's own bookkeeping would otherwise wait with vmcnt(0) on loads issued a moment earlier.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void ldg_untracked_nt(f32x4& d, const void* p) {
     asm volatile("global_load_dwordx4 %0, %1, off nt" : "+v"(d) : "v"(p));
 }
@@ -2956,6 +2969,22 @@ static int fwd_chunks(int64_t B, int64_t T, int64_t H, int64_t N, int64_t G, int
     return n;
 }
 
+// Batch rows of one group where a one-chunk forward runs as a pipeline over groups of whole batch rows (B: no
+// groups).  chain_fwd's LDS records let a round of its workgroups hold only so many chains; beyond that the rounds
+// follow each other anyway, so the replay of one group runs beside the chains of the next.  A group is at least
+// one round, and enough rounds of a short scan that its chains take about the 100 us that hide its launches.
+static int64_t fwd_group(int64_t B, int64_t T, int64_t H, int64_t N, int64_t D, int dtype) {
+    const int64_t NP = (N + 15) & ~15ll;
+    const size_t lds = D == 128 ? (dtype == SLOTSCAN_BF16 ? ChainLds<128, bf16_t>::bytes((int)NP) : ChainLds<128, float>::bytes((int)NP))
+                                : (dtype == SLOTSCAN_BF16 ? ChainLds<64, bf16_t>::bytes((int)NP) : ChainLds<64, float>::bytes((int)NP));
+    const int64_t round = 256 * std::max<int64_t>(1, 163840 / (int64_t)lds);
+    const int64_t chains = round * std::max<int64_t>(1, 192 / T);
+    if (B * H <= chains) return B;
+    int64_t g = std::max<int64_t>(1, chains / H);
+    g = std::max<int64_t>(g, (B + FWD_MAX_CHUNKS - 2) / (FWD_MAX_CHUNKS - 1));
+    return std::min<int64_t>(B, g);
+}
+
 static int check_q(int bits, int64_t group, int64_t D, bool codes) {
     if (codes ? (bits < 2 || bits > 8) : (bits != 0 && (bits < 2 || bits > 8)))
         return fail(SLOTSCAN_ERR_SHAPE, codes ? "bits must be 2..8" : "bits must be 0 or 2..8");
@@ -2995,7 +3024,7 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
     const bool f32 = mode == FE_F32;
     // the register-resident chain: built for D = 128 and more than 96 rows, where chain_fwd's records leave room for
     // one workgroup on each of the 256 CUs
-    const bool reg = f32 && nch > 1 && D == 128 && N > 96 && B * H > 256;
+    const bool reg = f32 && D == 128 && N > 96 && B * H > 256;
     ChainFwdArgs ca{q, k, gate, fr, temp, k0, o0, am, oold, cslog, kfin, ofin, (int)T, (int)H, (int)N, eps,
                     fr_per_token ? 1 : 0, occ_bin ? 1 : 0, 0, (int)T, o.kbuf, kold, (int)G, NB, (int)H, (int)H, 0};
     RowsFwdArgs ra{k, v, gate, am, k0, v0, nullptr, vfin, kold, vold, (int)T, (int)H, (int)N, (int)G, NB, 0, (int)T,
@@ -3009,17 +3038,46 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
     // already be overwriting kfin while the replay of an earlier chunk runs): with fp32 snapshots through the
     // snapshot of the next block, te / G, which is exactly the state there -- a chunk ends by writing it and
     // the next starts from it without storing it again -- else through kcarry and vfin.
+    // A scan of one chunk whose chains are more than a round of workgroups runs the same way over groups of whole
+    // batch rows (B 256, T 256, H 6, forward: bf16 copies at N 192 1,910 -> 1,575 us, at N 96 1,091 -> 1,037; fp32 at N 96 1,497 -> 1,385).
+    const int64_t gb = nch == 1 && !reg ? fwd_group(B, T, H, N, D, dtype) : B;
+    const int ng = (int)((B + gb - 1) / gb), nst = nch * ng;
     hipStream_t side = nullptr;
     hipEvent_t* ev = nullptr;
-    if (nch > 1)
-        if (int r = slothost::side_stream(&side, &ev, nch + 1)) return r;
-    const dim3 grid((unsigned)(B * H), (unsigned)((N + 31) / 32)), block(512);
+    if (nst > 1)
+        if (int r = slothost::side_stream(&side, &ev, nst + 1)) return r;
+    const dim3 block(512);
     hipError_t e;
-    for (int c = 0; c < nch; c++) {
-        ca.ts = ra.ts = (int)cb[c];
-        ca.te = ra.te = (int)cb[c + 1];
+    const ChainFwdArgs ca0 = ca;
+    const RowsFwdArgs ra0 = ra;
+    for (int c = 0; c < nst; c++) {
+        const int64_t b0 = ng > 1 ? c * gb : 0, Bg = ng > 1 ? std::min<int64_t>(gb, B - b0) : B;
+        const dim3 grid((unsigned)(Bg * H), (unsigned)((N + 31) / 32));
+        if (ng > 1) {                                    // the group's part of every tensor
+            const int64_t th = b0 * T * H, hn = b0 * H * N, sn = b0 * NB * H * N;
+            const int64_t esz = dtype == SLOTSCAN_BF16 ? 2 : 4;
+            auto at = [](auto* p, int64_t off) { return p ? p + off : p; };
+            auto tok = [&](const void* p) { return (const void*)((const char*)p + th * D * esz); };
+            ca.q = tok(ca0.q); ca.k = tok(ca0.k); ca.gate = ca0.gate + th; ca.fr = ca0.frt ? ca0.fr + th : ca0.fr;
+            ca.k0 = at(ca0.k0, hn * D); ca.o0 = at(ca0.o0, hn);
+            ca.am = ca0.am + th; ca.oold = at(ca0.oold, th); ca.cslog = at(ca0.cslog, b0 * H * T * N);
+            ca.kfin = ca0.kfin + hn * D; ca.ofin = ca0.ofin + hn;
+            ra.k = tok(ra0.k); ra.v = tok(ra0.v); ra.gate = ca.gate; ra.am = ca.am;
+            ra.k0 = at(ra0.k0, hn * D); ra.v0 = at(ra0.v0, hn * D);
+            ra.vfin = ra0.vfin + hn * D;
+            ra.kold = at(ra0.kold, th * D); ra.vold = at(ra0.vold, th * D);
+            ra.kbuf = at(ra0.kbuf, sn * D); ra.vbuf = at(ra0.vbuf, sn * D);
+            ra.kbm = at(ra0.kbm, sn * D); ra.vbm = at(ra0.vbm, sn * D);
+            ra.kinvm = at(ra0.kinvm, sn); ra.validm = at(ra0.validm, sn);
+            ra.kcode = at(ra0.kcode, sn * D); ra.vcode = at(ra0.vcode, sn * D);
+            const int64_t spr = ra0.kscale ? D / ra0.group : 0;
+            ra.kscale = at(ra0.kscale, sn * spr); ra.vscale = at(ra0.vscale, sn * spr);
+        }
+        const int ch = ng > 1 ? 0 : c;
+        ca.ts = ra.ts = (int)cb[ch];
+        ca.te = ra.te = (int)cb[ch + 1];
         const bool inner_end = ca.te < T;
-        if (c > 0) {
+        if (ch > 0) {
             ca.o0 = ofin;
             ca.k0 = reg ? o.kbuf + (size_t)(ca.ts / G) * H * N * D : kfin;
             if (f32) {
@@ -3036,7 +3094,7 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
         }
         if (f32) {
             ra.kfin = inner_end ? o.kbuf + (size_t)(ra.te / G) * H * N * D : nullptr;
-            ra.vfin = inner_end ? o.vbuf + (size_t)(ra.te / G) * H * N * D : vfin;
+            if (nch > 1) ra.vfin = inner_end ? o.vbuf + (size_t)(ra.te / G) * H * N * D : vfin;
             ra.kfbs = ra.vfbs = inner_end ? NB * (int)H : (int)H;
             if (reg) {                                   // the chain writes and carries the keys' snapshots itself
                 ca.kfin = inner_end ? ra.kfin : kfin;
@@ -3047,16 +3105,16 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
         }
         {
             slothost::Scope sc(SLOTSCAN_K_CHAIN_FWD, st);
-            if (D == 128) e = dtype == SLOTSCAN_BF16 ? launch_chain_fwd<128, bf16_t>(ca, (int)B, reg, st) : launch_chain_fwd<128, float>(ca, (int)B, reg, st);
-            else e = dtype == SLOTSCAN_BF16 ? launch_chain_fwd<64, bf16_t>(ca, (int)B, reg, st) : launch_chain_fwd<64, float>(ca, (int)B, reg, st);
+            if (D == 128) e = dtype == SLOTSCAN_BF16 ? launch_chain_fwd<128, bf16_t>(ca, (int)Bg, reg, st) : launch_chain_fwd<128, float>(ca, (int)Bg, reg, st);
+            else e = dtype == SLOTSCAN_BF16 ? launch_chain_fwd<64, bf16_t>(ca, (int)Bg, reg, st) : launch_chain_fwd<64, float>(ca, (int)Bg, reg, st);
         }
         if (e != hipSuccess) return hip_fail(e, "chain_fwd launch");
         hipStream_t rs = st;
-        if (nch > 1 && c + 1 < nch) {
+        if (nst > 1 && c + 1 < nst) {
             if ((e = hipEventRecord(ev[c], st)) != hipSuccess) return hip_fail(e, "hipEventRecord");
             if ((e = hipStreamWaitEvent(side, ev[c], 0)) != hipSuccess) return hip_fail(e, "hipStreamWaitEvent");
             rs = side;
-        } else if (nch > 1) {
+        } else if (nst > 1) {
             // the last chunk's replay follows its chain on the caller's stream, behind the side stream's
             // replays (its value carry): no cross-stream wait between the chain and it, and no join after it
             if ((e = hipEventRecord(ev[c], side)) != hipSuccess) return hip_fail(e, "hipEventRecord");
