@@ -38,9 +38,28 @@ inline void launch(F kernel, const dim3& grid, const dim3& block, uint32_t shm, 
 
 inline bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
-// The library's second stream on the current device (non-blocking, default priority) and a pool of
-// timing-free events, for fork/join pipelines inside one entry point.  Created on first use per device and
-// kept until the process ends.  Returns 0, or SLOTSCAN_ERR_HIP with the message set.
-int side_stream(hipStream_t* side, hipEvent_t** ev, int nev);
+// One fork/join section of an entry point: a second stream (non-blocking, default priority) and events of the current
+// device, held by this section alone while it enqueues -- host threads enqueue at the same time, and an event that
+// another call records again between this call's record and its wait would let a kernel run before its input is
+// there.  The sets are kept for later sections until the process ends, one for each section that was ever open at
+// the same time; a set whose stream still belongs to another graph capture is passed over.
+struct ForkSet;
+class Fork {
+public:
+    Fork() = default;
+    Fork(const Fork&) = delete;
+    Fork& operator=(const Fork&) = delete;
+    ~Fork();                                             // gives the set back
+    // Take a set with `nev` events.  Returns 0, or SLOTSCAN_ERR_HIP with the message set.
+    int open(hipStream_t caller, int nev);
+    // The second stream waits for what the caller's stream holds, and the other way round (event i of the set).
+    hipError_t fork(int i);
+    hipError_t join(int i);
+    hipStream_t side() const;
+private:
+    ForkSet* set_ = nullptr;
+    hipStream_t caller_ = nullptr;
+    int dev_ = 0;
+};
 
 }  // namespace slothost

@@ -2789,6 +2789,7 @@ hipError_t launch_chain_bwd(const ChainBwdArgs& a, int B, hipStream_t st) {
 #include "slotscan.h"
 #include <algorithm>
 #include <mutex>
+#include <new>
 #include <vector>
 
 // Optional per-kernel timing with HIP events recorded on the launch stream around every kernel (the
@@ -2838,28 +2839,63 @@ Scope::~Scope() {
     }
 }
 
-static std::mutex side_mu;
-struct SideRes { hipStream_t s = nullptr; std::vector<hipEvent_t> ev; };
-static SideRes side_res[64];
-int side_stream(hipStream_t* side, hipEvent_t** ev, int nev) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+constexpr int FORK_EVENTS = 48;
+struct ForkSet { hipStream_t side; hipEvent_t ev[FORK_EVENTS]; int nev; ForkSet* next; };
+static std::mutex fork_mu;
+static ForkSet* fork_free[64];                          // per device: the sets that no section holds
+
+// Whether a section on `caller` may use the set: its stream is in no capture, or in the caller's own.
+static bool fork_usable(const ForkSet* s, hipStream_t caller) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone, cst = hipStreamCaptureStatusNone;
+    unsigned long long id = 0, cid = 0;
+    if (hipStreamGetCaptureInfo(s->side, &st, &id) != hipSuccess) { (void)hipGetLastError(); return false; }
+    if (st == hipStreamCaptureStatusNone) return true;
+    if (hipStreamGetCaptureInfo(caller, &cst, &cid) != hipSuccess) { (void)hipGetLastError(); return false; }
+    return st == hipStreamCaptureStatusActive && cst == st && cid == id;
+}
+int Fork::open(hipStream_t caller, int nev) {
+    hipError_t e = hipGetDevice(&dev_);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-    if (dev < 0 || dev >= 64) return fail(SLOTSCAN_ERR_HIP, "device id out of range");
-    std::lock_guard<std::mutex> g(side_mu);
-    SideRes& r = side_res[dev];
-    if (!r.s && (e = hipStreamCreateWithFlags(&r.s, hipStreamNonBlocking)) != hipSuccess) {
-        r.s = nullptr;
-        return hip_fail(e, "hipStreamCreateWithFlags");
+    if (dev_ < 0 || dev_ >= 64) return fail(SLOTSCAN_ERR_HIP, "device id out of range");
+    if (nev > FORK_EVENTS) return fail(SLOTSCAN_ERR_HIP, "too many events in one section");
+    caller_ = caller;
+    {
+        std::lock_guard<std::mutex> g(fork_mu);
+        for (ForkSet** p = &fork_free[dev_]; *p; p = &(*p)->next)
+            if (fork_usable(*p, caller)) {
+                set_ = *p;
+                *p = set_->next;
+                break;
+            }
     }
-    while ((int)r.ev.size() < nev) {
-        hipEvent_t x = nullptr;
-        if ((e = hipEventCreateWithFlags(&x, hipEventDisableTiming)) != hipSuccess) return hip_fail(e, "hipEventCreate");
-        r.ev.push_back(x);
+    if (!set_) {
+        hipStream_t s = nullptr;
+        if ((e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking)) != hipSuccess) return hip_fail(e, "hipStreamCreateWithFlags");
+        set_ = new (std::nothrow) ForkSet{s, {}, 0, nullptr};
+        if (!set_) {
+            (void)hipStreamDestroy(s);
+            return fail(SLOTSCAN_ERR_HIP, "out of host memory");
+        }
     }
-    *side = r.s;
-    *ev = r.ev.data();
+    for (; set_->nev < nev; set_->nev++)
+        if ((e = hipEventCreateWithFlags(&set_->ev[set_->nev], hipEventDisableTiming)) != hipSuccess)
+            return hip_fail(e, "hipEventCreate");
     return 0;
+}
+hipStream_t Fork::side() const { return set_->side; }
+hipError_t Fork::fork(int i) {
+    const hipError_t e = hipEventRecord(set_->ev[i], caller_);
+    return e != hipSuccess ? e : hipStreamWaitEvent(set_->side, set_->ev[i], 0);
+}
+hipError_t Fork::join(int i) {
+    const hipError_t e = hipEventRecord(set_->ev[i], set_->side);
+    return e != hipSuccess ? e : hipStreamWaitEvent(caller_, set_->ev[i], 0);
+}
+Fork::~Fork() {
+    if (!set_) return;
+    std::lock_guard<std::mutex> g(fork_mu);
+    set_->next = fork_free[dev_];
+    fork_free[dev_] = set_;
 }
 
 static thread_local char g_err[512];
@@ -2936,6 +2972,7 @@ static int64_t fwd_chunk_len(int64_t T, int64_t G) {
 // the tail the replay leaves exposed (the last chunk's) and the number of chunk starts are both small, while
 // each replay still hides behind the next chain chunk, half as long.
 #define FWD_MAX_CHUNKS 40
+static_assert(FWD_MAX_CHUNKS <= slothost::FORK_EVENTS, "a forward holds an event per chunk");
 static int fwd_chunks(int64_t B, int64_t T, int64_t H, int64_t N, int64_t G, int64_t* b) {
     b[0] = 0;
     const int64_t len = fwd_chunk_len(T, G);
@@ -3042,10 +3079,9 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
     // batch rows (B 256, T 256, H 6, forward: bf16 copies at N 192 1,910 -> 1,575 us, at N 96 1,091 -> 1,037; fp32 at N 96 1,497 -> 1,385).
     const int64_t gb = nch == 1 && !reg ? fwd_group(B, T, H, N, D, dtype) : B;
     const int ng = (int)((B + gb - 1) / gb), nst = nch * ng;
-    hipStream_t side = nullptr;
-    hipEvent_t* ev = nullptr;
+    slothost::Fork fk;
     if (nst > 1)
-        if (int r = slothost::side_stream(&side, &ev, nst + 1)) return r;
+        if (int r = fk.open(st, nst)) return r;
     const dim3 block(512);
     hipError_t e;
     const ChainFwdArgs ca0 = ca;
@@ -3111,14 +3147,12 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
         if (e != hipSuccess) return hip_fail(e, "chain_fwd launch");
         hipStream_t rs = st;
         if (nst > 1 && c + 1 < nst) {
-            if ((e = hipEventRecord(ev[c], st)) != hipSuccess) return hip_fail(e, "hipEventRecord");
-            if ((e = hipStreamWaitEvent(side, ev[c], 0)) != hipSuccess) return hip_fail(e, "hipStreamWaitEvent");
-            rs = side;
+            if ((e = fk.fork(c)) != hipSuccess) return hip_fail(e, "fork");
+            rs = fk.side();
         } else if (nst > 1) {
             // the last chunk's replay follows its chain on the caller's stream, behind the side stream's
             // replays (its value carry): no cross-stream wait between the chain and it, and no join after it
-            if ((e = hipEventRecord(ev[c], side)) != hipSuccess) return hip_fail(e, "hipEventRecord");
-            if ((e = hipStreamWaitEvent(st, ev[c], 0)) != hipSuccess) return hip_fail(e, "hipStreamWaitEvent");
+            if ((e = fk.join(c)) != hipSuccess) return hip_fail(e, "join");
         }
         {
             slothost::Scope sc(SLOTSCAN_K_ROWS_FWD, rs);

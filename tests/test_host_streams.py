@@ -1,0 +1,113 @@
+"""CPU checks of what the forward's host code enqueues: the library runs against a stand-in for the HIP runtime
+(hip_stub.c) that records launches, event records and waits instead of executing them."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+import slotscan_lib as L
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+# Runs in its own process, which never loads the real runtime.  `call(thread, stream, **shape)` is one slotscan_fwd.
+_PRELUDE = """
+import ctypes, json, sys, threading
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+stub.stub_log.restype = ctypes.c_char_p
+stub.stub_capture.argtypes = [ctypes.c_void_p, ctypes.c_uint64]
+lib = ctypes.CDLL(sys.argv[2])
+vp, i64, i32, f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
+lib.slotscan_fwd.argtypes = [vp, vp, vp, i32, vp, vp, i32, vp] + [i64] * 6 + [f32, i32] + [vp] * 14
+def call(thread, stream, B=8, T=1024, H=6, N=192, D=128, G=8):
+    stub.stub_thread(thread)
+    p = 1 << 20
+    return lib.slotscan_fwd(p, p, p, 1, p, p, 1, p, B, T, H, N, D, G, 1e-4, 1, None, None, None, p, p, p, None, None, None,
+                            None, p, p, p, stream)
+def log():
+    return [l.split() for l in stub.stub_log().decode().splitlines()]
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    d = tmp_path_factory.mktemp("hip_stub")
+    out, ver = str(d / "libamdhip64.so.7"), str(d / "version.map")
+    with open(ver, "w") as f:
+        f.write("hip_4.2 { global: *; };\nhip_4.5 { global: hipStreamGetCaptureInfo; };\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-pthread", os.path.join(HERE, "hip_stub.c"), "-o", out,
+                    "-Wl,-soname,libamdhip64.so.7", "-Wl,--version-script=" + ver], check=True)
+    return out
+
+
+def _run(stub, body):
+    r = subprocess.run([sys.executable, "-c", _PRELUDE + body, stub, L.LIB_PATH], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return json.loads(r.stdout.splitlines()[-1])
+
+
+def _check_waits(log):
+    """Every wait of a call is for an event that the same call recorded last."""
+    last = {}
+    n = 0
+    for op in log:
+        if op[1] == "record":
+            last[op[2]] = op[0]
+        elif op[1] == "wait":
+            n += 1
+            assert last.get(op[3]) == op[0], f"a wait of call {op[0]} is for call {last.get(op[3])}'s record"
+    return n
+
+
+@pytest.mark.parametrize("shape", [dict(B=8, T=1024),                       # chunks of a long scan
+                                   dict(B=600, T=200, H=1, N=70)])          # batch groups of a short one
+def test_two_threads_keep_their_own_events(stub, shape):
+    """Two host threads inside the forward on one device: neither takes the other's events, also when one is stopped
+    between a record and its wait while the other records."""
+    log = _run(stub, f"""
+stub.stub_hold(1, 2)
+rc = [None, None, None]
+def go(i):
+    rc[i] = call(i, 0x100 * i, **{shape!r})
+a, b = threading.Thread(target=go, args=(1,)), threading.Thread(target=go, args=(2,))
+a.start(); b.start(); a.join(); b.join()
+assert rc[1:] == [0, 0], rc
+print(json.dumps(log()))
+""")
+    assert _check_waits(log) >= 4
+    for i in ("1", "2"):                                # and each call ends with its replays joined to its stream
+        mine = [op for op in log if op[0] == i]
+        side = {op[3] for op in mine if op[1] == "launch"} - {hex(0x100 * int(i))}
+        assert len(side) == 1
+        last_side = max(k for k, op in enumerate(mine) if op[1] == "launch" and op[3] in side)
+        joined = [k for k, op in enumerate(mine) if op[1] == "record" and op[3] in side and k > last_side]
+        assert joined and any(op[1] == "wait" and op[2] == hex(0x100 * int(i)) and op[3] == mine[joined[0]][2]
+                              for op in mine[joined[0]:])
+
+
+def test_a_set_held_by_another_capture_is_passed_over(stub):
+    """While the second stream of an earlier call belongs to a graph capture, a call outside that capture takes another
+    one; a call of the same capture may take it, and no third one is made."""
+    side = lambda log, st: {op[3] for op in log if op[1] == "launch"} - {hex(st)}
+    a, b, c, d = _run(stub, """
+out = []
+def one(stream):
+    stub.stub_reset()
+    assert call(1, stream) == 0
+    return log()
+out.append(one(0x100))
+side = ({op[3] for op in out[0] if op[1] == "launch"} - {"0x100"}).pop()
+stub.stub_capture(int(side, 16), 7)
+stub.stub_capture(0x100, 7)
+out.append(one(0x200))
+out.append(one(0x100))
+stub.stub_capture(int(side, 16), 0)
+stub.stub_capture(0x100, 0)
+out.append(one(0x200))
+print(json.dumps(out))
+""")
+    assert len(side(a, 0x100)) == 1 and not side(b, 0x200) & side(a, 0x100)
+    assert side(c, 0x100) | side(d, 0x200) <= side(a, 0x100) | side(b, 0x200)
+    for log in (a, b, c, d):
+        _check_waits(log)
