@@ -49,7 +49,7 @@ public:
     Fork() = default;
     Fork(const Fork&) = delete;
     Fork& operator=(const Fork&) = delete;
-    ~Fork();                                             // gives the set back
+    ~Fork();                                             // joins what is not joined yet (an early return), gives the set back
     // Take a set with `nev` events.  Returns 0, or SLOTSCAN_ERR_HIP with the message set.
     int open(hipStream_t caller, int nev);
     // The second stream waits for what the caller's stream holds, and the other way round (event i of the set).
@@ -60,6 +60,7 @@ private:
     ForkSet* set_ = nullptr;
     hipStream_t caller_ = nullptr;
     int dev_ = 0;
+    bool ahead_ = false;                                 // the second stream may hold work that the caller's does not wait for
 };
 
 }  // namespace slothost

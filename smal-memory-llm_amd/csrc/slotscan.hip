@@ -2885,14 +2885,18 @@ int Fork::open(hipStream_t caller, int nev) {
 hipStream_t Fork::side() const { return set_->side; }
 hipError_t Fork::fork(int i) {
     const hipError_t e = hipEventRecord(set_->ev[i], caller_);
+    ahead_ = true;
     return e != hipSuccess ? e : hipStreamWaitEvent(set_->side, set_->ev[i], 0);
 }
 hipError_t Fork::join(int i) {
-    const hipError_t e = hipEventRecord(set_->ev[i], set_->side);
-    return e != hipSuccess ? e : hipStreamWaitEvent(caller_, set_->ev[i], 0);
+    hipError_t e = hipEventRecord(set_->ev[i], set_->side);
+    if (e == hipSuccess) e = hipStreamWaitEvent(caller_, set_->ev[i], 0);
+    if (e == hipSuccess) ahead_ = false;
+    return e;
 }
 Fork::~Fork() {
     if (!set_) return;
+    if (ahead_) (void)join(0);
     std::lock_guard<std::mutex> g(fork_mu);
     set_->next = fork_free[dev_];
     fork_free[dev_] = set_;

@@ -111,3 +111,18 @@ print(json.dumps(out))
     assert side(c, 0x100) | side(d, 0x200) <= side(a, 0x100) | side(b, 0x200)
     for log in (a, b, c, d):
         _check_waits(log)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4])
+def test_a_failed_launch_leaves_nothing_unjoined(stub, n):
+    """A call that fails half way still joins what it put on the second stream: the caller may free or reuse the buffers
+    in its own stream's order."""
+    log = _run(stub, f"""
+stub.stub_fail_launch({n})
+assert call(1, 0x100) != 0
+print(json.dumps(log()))
+""")
+    side = [k for k, op in enumerate(log) if op[1] == "launch" and op[3] != "0x100"]
+    assert sum(op[1] == "launch" for op in log) == n + 1 and side
+    joined = [k for k, op in enumerate(log) if op[1] == "record" and op[3] == log[side[0]][3] and k > side[-1]]
+    assert joined and any(op[1] == "wait" and op[2] == "0x100" and op[3] == log[joined[0]][2] for op in log[joined[0]:])
