@@ -994,19 +994,23 @@ void chain_fwd(ChainFwdArgs a) {
                 e1 = en;
 #pragma unroll
                 for (int e = 0; e < EPL; e++) kv[e] = kn_[e];
-                // the row's occupancy crossed eps (its first write), or the scores take the occupancy itself
-                const u32 cross = (u32)(__ballot(sn >= eps) ^ __ballot(so >= eps));
-                if (__builtin_expect((cross & (1u << CT)) || !occb, 0)) {
+                // the row's occupancy crossed eps (its first write), or the scores take the occupancy itself; one branch,
+                // because every step of the chain waits for it
+                const u32 cross = (u32)(__ballot(sn >= eps) ^ __ballot(so >= eps)) & (1u << CT);
+                if (__builtin_expect(cross || !occb, 0)) {
                     const float on = readlanef(sn, CT);
                     const bool now = on >= eps;
-                    const int al = am / NR, ar = am - NR * al;
 #pragma unroll
-                    for (int r = 0; r < NR; r++) {
-                        const u64 bit = ar == r ? 1ull << al : 0ull;
-                        tk[r] = now ? tk[r] | bit : tk[r] & ~bit;
-                        oc[r] = n0 + r == am ? (occb ? (now ? 1.f : 0.f) : on) : oc[r];
+                    for (int r = 0; r < NR; r++) oc[r] = n0 + r == am ? (occb ? (now ? 1.f : 0.f) : on) : oc[r];
+                    if (cross) {                         // other rows compete from the next step on
+                        const int al = am / NR, ar = am - NR * al;
+#pragma unroll
+                        for (int r = 0; r < NR; r++) {
+                            const u64 bit = ar == r ? 1ull << al : 0ull;
+                            tk[r] = now ? tk[r] | bit : tk[r] & ~bit;
+                        }
+                        compete();
                     }
-                    compete();
                 }
             };
             // four steps a turn: constant offsets inside it, and code that stays a small part of the instruction

@@ -42,16 +42,18 @@ def test_chain_one_competing_row(N, T):
         assert abs(np64(got) - ref).max() <= 1e-5 * max(abs(ref).max(), 1e-30)
 
 
-def test_chain_occupancy_next_to_the_threshold():
-    """Gates around eps: rows whose first writes leave them free, and exact zeros and ones."""
+@pytest.mark.parametrize("occb", [True, False])
+def test_chain_occupancy_next_to_the_threshold(occb):
+    """Gates around eps: rows whose first writes leave them free, and exact zeros and ones.  Without occ_bin the scores take
+    the occupancy of every write, while the rows that compete change only where one crosses the threshold."""
     B, T, H, N, D = 2, 80, 2, 24, 64
     k, q, v, g, fr = scan_inputs(B, T, H, D, 500, gate_mix=True)
     g = torch.where(torch.rand(B, T, H, generator=torch.Generator().manual_seed(7)) < 0.5, g * 1.5e-4, g)
     run = lambda lo, hi, st: KH.kv_scan_stream(*(x[:, lo:hi].cuda() for x in (k, v, g, fr)), N, 16.0, G=8,
-                                               q=q[:, lo:hi].cuda(), occ_bin=True, state=st)
+                                               q=q[:, lo:hi].cuda(), occ_bin=occb, state=st)
     kb, vb, st = run(0, T, None)
     okb, ovb, info = SO.scan_forward(np64(k), np64(v), np64(g), np64(fr), N, 16.0, G=8, hard=True, q=np64(q),
-                                     occ_bin=True)
+                                     occ_bin=occb)
     # every value of the state is a blend of at most T unit-scale tokens in fp32: 1e-5 of the largest
     for got, ref in ((kb, okb), (vb, ovb), (st[2].reshape(B, H, N), info["ofin"])):
         assert abs(np64(got) - ref).max() <= 1e-5 * abs(ref).max()
