@@ -234,9 +234,9 @@ struct ChainFwdArgs {
     int32_t* am; float* oold; float* cslog; float* kfin; float* ofin;
     int T, H, N; float eps; int frt, occb;
     int ts, te;                                          // steps [ts, te) of the T-long sequence
-    // chain_fwd_reg: the fp32 snapshots and the old key rows it writes, and, as RowsFwdArgs, the slabs it starts
-    // from and ends in
-    float* kbuf; float* kold;
+    // chain_fwd_reg: the copies (kbuf, or kbm with kinv and valid, or none) and the old key rows that it writes, and, as
+    // RowsFwdArgs, the slabs it starts from and ends in
+    float* kbuf; bf16_t* kbm; float* kinvm; uint8_t* validm; float* kold;
     int G, NB, k0bs, kfbs, skip0;
 };
 
@@ -261,6 +261,17 @@ __device__ __forceinline__ void st_slice_at(float* base, u32 boff, const float* 
     }
 }
 
+// The same slice as bf16 (the writer epilogue's cast, round to nearest even): 8 bytes per 4 elements
+template <int EPL>
+__device__ __forceinline__ void st_slice_bf_at(bf16_t* base, u32 boff, const float* s) {
+    char* p = reinterpret_cast<char*>(base) + boff;
+#pragma unroll
+    for (int jj = 0; jj < EPL / 4; jj++) {
+        const u32x2 r = {pack_bf16x2(s[4 * jj], s[4 * jj + 1]), pack_bf16x2(s[4 * jj + 2], s[4 * jj + 3])};
+        __builtin_nontemporal_store(r, reinterpret_cast<u32x2*>(p + 128 * jj));
+    }
+}
+
 // Wave max of an ordered key (fkey), at every lane: integer max needs no NaN canonicalisation, so each
 // DPP stage is one v_max_u32 with a DPP source.
 __device__ __forceinline__ u32 wavemax_key(u32 v) {
@@ -274,10 +285,12 @@ __device__ __forceinline__ u32 wavemax_key(u32 v) {
     return max(r[0], r[1]);
 }
 
-// The key chain with its keys in registers, which also writes the fp32 key snapshots.  It serves the fp32 contract
-// where the chains are more than one round of chain_fwd's workgroups (below): the forward is then bound by its
-// snapshot bytes, and this kernel, half of a CU's registers a workgroup, holds twice the chains at once and writes
-// the keys' half of them while it steps, also where the replay has nothing to do yet.  H 6, N 192, D 128: B 64, T 1024
+// The key chain with its keys in registers, which emits the keys' copies itself as it steps: the fp32 snapshots, or the
+// writer epilogue's bf16 copies with kinv and valid (CR_NONE: the row replay emits them).  fwd_chain_reg says where it
+// runs instead of chain_fwd (below).  A step takes three times as long, but a workgroup takes half of a CU's
+// registers, so twice the chains run at once, and it starts sooner.  With fp32 snapshots the forward is bound by
+// their bytes, and this kernel writes the keys' half of them while it steps, also where the replay has nothing to do
+// yet.  H 6, N 192, D 128, fp32 snapshots: B 64, T 1024
 // forward and backward 4.96 ms against 5.09 ms with chain_fwd; B 256, T 256 forward 2.29 against 2.77 ms; B 64, T 256
 // 0.67 against 0.77 ms (N 96, one round, B 64, T 1024: 3.41 against 3.00 ms, and chain_fwd it is).
 //
@@ -298,7 +311,8 @@ __device__ __forceinline__ u32 wavemax_key(u32 v) {
 // the next window).  The row norm of the written row is recomputed from its new elements.  The per-step
 // work left is the score, the argmax, and the one-row update.
 #define REG_THREADS (CHAIN_THREADS + 64)
-template <int D, int P, typename TI>
+enum { CR_NONE = 0, CR_F32 = 1, CR_BF = 2 };             // what it emits of the keys (RowsFwdArgs' buffers)
+template <int D, int P, typename TI, int EM>
 __global__ __attribute__((amdgpu_flat_work_group_size(REG_THREADS, REG_THREADS), amdgpu_waves_per_eu(2)))
 void chain_fwd_reg(ChainFwdArgs a) {
     constexpr int EPL = D / 16;
@@ -415,9 +429,13 @@ void chain_fwd_reg(ChainFwdArgs a) {
     const ChainRows<P> R(tid);
     const size_t sstride = (size_t)H * N * D;
     const size_t snap0 = ((size_t)b * a.NB + ts / G) * H + h;           // (b, ts / G, h): snapshot of block ts / G
-    float* kb = a.kbuf + snap0 * N * D + (a.skip0 ? sstride : 0);   // skip0: the first slab is written
+    float* kb = EM == CR_F32 ? a.kbuf + snap0 * N * D + (a.skip0 ? sstride : 0) : nullptr;   // skip0: the first slab is written
+    bf16_t* kbm = EM == CR_BF ? a.kbm + snap0 * N * D : nullptr;
+    float* kinvm = EM == CR_BF ? a.kinvm + snap0 * N : nullptr;
+    uint8_t* validm = EM == CR_BF ? a.validm + snap0 * N : nullptr;
     rowv Kv[EPL];                                       // Kv[e][j]: element e of this lane's slice of row j
     float o_me = 0.f, kinv_me;
+    bool vld_me;                                        // |K_me|^2 > 1e-12 (the epilogue's `valid`)
     {
         // the P rows' loads go out together (from row min(n, N - 1), unconditionally) and rows past N are
         // zeroed afterwards: a load per row behind a branch, used right away, waited for each row in turn
@@ -458,6 +476,7 @@ void chain_fwd_reg(ChainFwdArgs a) {
             nsq0 = (c >> RS<P>::SH) == j ? sj : nsq0;
         }
         kinv_me = rsq_clamped(nsq0);
+        vld_me = nsq0 > 1e-12f;
         if (a.o0 && R.n_me < N) o_me = a.o0[(size_t)bh * N + R.n_me];
     }
     auto row_of = [&](int j, float* row) {
@@ -554,7 +573,7 @@ void chain_fwd_reg(ChainFwdArgs a) {
             uint4 r[CHAIN_WAVES];
 #pragma unroll
             for (int w = 0; w < CHAIN_WAVES; w++) r[w] = s_red[par][w];
-            if (gc == 0 && (t != ts || !a.skip0)) {   // the PRE-write key state of block t / G:
+            if (EM != CR_NONE && gc == 0 && (EM == CR_BF || t != ts || !a.skip0)) {   // the PRE-write key state of block t / G:
                 u32 ro = roff;                              // every row group stores whole rows
                 int nvv = nvalid;
                 asm volatile("" : "+v"(ro), "+v"(nvv));     // per-snapshot offsets, not 16 live registers
@@ -562,9 +581,22 @@ void chain_fwd_reg(ChainFwdArgs a) {
                 for (int jr = 0; jr < P; jr++) {
                     float row[EPL];
                     row_of(jr, row);
-                    if (jr < nvv) st_slice_at<EPL, true>(kb, ro + (u32)(jr * D * 4), row);
+                    if (jr < nvv) {
+                        if constexpr (EM == CR_BF) st_slice_bf_at<EPL>(kbm, (ro >> 1) + (u32)(jr * D * 2), row);
+                        else st_slice_at<EPL, true>(kb, ro + (u32)(jr * D * 4), row);
+                    }
                 }
-                kb += sstride;
+                if constexpr (EM == CR_BF) {
+                    if (R.prim && valid_me) {
+                        kinvm[R.n_me] = kinv_me;
+                        validm[R.n_me] = vld_me ? 1 : 0;
+                    }
+                    kbm += sstride;
+                    kinvm += (size_t)H * N;
+                    validm += (size_t)H * N;
+                } else {
+                    kb += sstride;
+                }
             }
             if (++gc == G) gc = 0;
             // waves in order = rows in order: strict '>' keeps the lowest row on ties
@@ -603,12 +635,13 @@ void chain_fwd_reg(ChainFwdArgs a) {
                 for (int e = 0; e < EPL; e++) Kv[e][sl] = nv[e];
 #pragma unroll
                 for (int e = 0; e < EPL; e++) part = fmaf(nv[e], nv[e], part);
-                if (a.kold) st_slice_nt<EPL>(a.kold + ix * D, old, c);
+                if (EM != CR_NONE && a.kold) st_slice_nt<EPL>(a.kold + ix * D, old, c);
                 const float kk = rowsum16(part);
                 if (R.n_me == amv) {
                     if (a.oold && R.prim) a.oold[ix] = o_me;
                     o_me = omw * o_me + g;
                     kinv_me = rsq_clamped(kk);
+                    vld_me = kk > 1e-12f;
                     // all 16 entries: those at or before step j are never read again in this window
 #pragma unroll
                     for (int q4 = 0; q4 < CT / 4; q4++)
@@ -1125,16 +1158,16 @@ __device__ __forceinline__ u32 pack_codes4(const float* cd) {
 // lane forms the mask of steps that wrote its row (4 LDS reads) and, with the piece's G-aligned snapshot
 // steps, walks the set bits in step order (snapshot first: it is the PRE-write state).
 // The key replay is the chain's own blend on the same token values, so bitwise the chain's keys.
-// EM: RF_F32 fp32 snapshots (RF_F32V: of the values alone, where the chain writes the keys'); RF_CODES the storage
-// quantiser's integer form; RF_MEM the writer epilogue's bf16 copies with kinv and valid, after the quantiser
-// where bits > 0.  The states cross the forward pipeline's inner chunk boundaries through kfin and vfin (each
+// EM: RF_F32 fp32 snapshots; RF_CODES the storage quantiser's integer form; RF_MEM the writer epilogue's bf16 copies
+// with kinv and valid, after the quantiser where bits > 0; RF_F32V, RF_MEMV the values' alone, where the chain emits
+// the keys'.  The states cross the forward pipeline's inner chunk boundaries through kfin and vfin (each
 // chunk's replay ends by writing them and the next starts from them), apart from the chain's own carry.
-enum { RF_F32 = 0, RF_CODES = 1, RF_MEM = 2, RF_F32V = 3 };
+enum { RF_F32 = 0, RF_CODES = 1, RF_MEM = 2, RF_F32V = 3, RF_MEMV = 4 };
 template <int D, typename TI, int EM>
 ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
     constexpr int EPL = D / 16;
     constexpr int NP = EPL / 4;
-    constexpr bool KR = EM != RF_F32V;                   // the key rows too
+    constexpr bool KR = EM != RF_F32V && EM != RF_MEMV;  // the key rows too
     constexpr int TC = 256;                              // staged steps: 2 KB of LDS, so the replay blocks fit beside a chain block on a CU
     __shared__ __align__(16) int s_am[TC];
     __shared__ float s_g[TC];
@@ -1181,10 +1214,12 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
 #pragma unroll
                 for (int e = 0; e < EPL; e++) { kv[e] = K[e]; vv[e] = V[e]; }
             }
-            float sq = 0.f;
+            if (KR) {
+                float sq = 0.f;
 #pragma unroll
-            for (int e = 0; e < EPL; e++) sq = fmaf(kv[e], kv[e], sq);
-            ks[0] = rowsum16(sq);
+                for (int e = 0; e < EPL; e++) sq = fmaf(kv[e], kv[e], sq);
+                ks[0] = rowsum16(sq);
+            }
 #pragma unroll
             for (int jj = 0; jj < NP; jj++) {
                 kx[jj] = u32x2{pack_bf16x2(kv[4 * jj], kv[4 * jj + 1]), pack_bf16x2(kv[4 * jj + 2], kv[4 * jj + 3])};
@@ -1197,7 +1232,7 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
                     const u32x2 rcv = {dppu<SLOT_DPP_XOR1>(snd.x), dppu<SLOT_DPP_XOR1>(snd.y)};
                     if (odd) x[0] = rcv; else x[1] = rcv;
                 };
-                trade(kx);
+                if (KR) trade(kx);
                 trade(vx);
             }
         }
@@ -1218,16 +1253,14 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
             }
         } else {
             const int o = NP == 2 ? (c & 1) * 128 + (c >> 1) * 16 : 8 * c;
-            char* kr = reinterpret_cast<char*>(a.kbm + srow * D) + o;
-            char* vr = reinterpret_cast<char*>(a.vbm + srow * D) + o;
-            if constexpr (NP == 2) {                     // 16 bytes a lane
-                __builtin_nontemporal_store(u32x4{kx[0].x, kx[0].y, kx[NP - 1].x, kx[NP - 1].y}, reinterpret_cast<u32x4*>(kr));
-                __builtin_nontemporal_store(u32x4{vx[0].x, vx[0].y, vx[NP - 1].x, vx[NP - 1].y}, reinterpret_cast<u32x4*>(vr));
-            } else {
-                __builtin_nontemporal_store(kx[0], reinterpret_cast<u32x2*>(kr));
-                __builtin_nontemporal_store(vx[0], reinterpret_cast<u32x2*>(vr));
-            }
-            if (c == 0) {                                // kinv and valid of the emitted (quantised) keys
+            auto put = [&](bf16_t* to, const u32x2* x) {
+                char* r = reinterpret_cast<char*>(to + srow * D) + o;
+                if constexpr (NP == 2) __builtin_nontemporal_store(u32x4{x[0].x, x[0].y, x[NP - 1].x, x[NP - 1].y}, reinterpret_cast<u32x4*>(r));
+                else __builtin_nontemporal_store(x[0], reinterpret_cast<u32x2*>(r));
+            };
+            if (KR) put(a.kbm, kx);
+            put(a.vbm, vx);
+            if (KR && c == 0) {                                // kinv and valid of the emitted (quantised) keys
                 a.kinvm[srow] = rsqrtf(fmaxf(ks[0], 1e-12f));
                 a.validm[srow] = ks[0] > 1e-12f ? 1 : 0;
             }
@@ -2737,13 +2770,15 @@ __global__ __launch_bounds__(256) void reduce_parts(const float* __restrict__ pa
 // ===================================================================================== host dispatch
 template <int D, typename TI>
 hipError_t launch_chain_fwd(const ChainFwdArgs& a, int B, bool reg, hipStream_t st) {
-    if constexpr (D == 128) {
-        if (reg) {
-            slothost::launch((chain_fwd_reg<D, 16, TI>), dim3(B * a.H), dim3(REG_THREADS), 0, st, a);
-            return hipGetLastError();
-        }
-    }
     const dim3 grid(B * a.H), block(FWD_THREADS);
+    if (reg) {
+#define SLOT_CR(PP) { if (a.kbuf) slothost::launch((chain_fwd_reg<D, PP, TI, CR_F32>), grid, dim3(REG_THREADS), 0, st, a); \
+                      else if (a.kbm) slothost::launch((chain_fwd_reg<D, PP, TI, CR_BF>), grid, dim3(REG_THREADS), 0, st, a); \
+                      else slothost::launch((chain_fwd_reg<D, PP, TI, CR_NONE>), grid, dim3(REG_THREADS), 0, st, a); }
+        if (a.N <= 8 * 4 * CHAIN_WAVES) SLOT_CR(8) else SLOT_CR(16)
+#undef SLOT_CR
+        return hipGetLastError();
+    }
     const uint32_t lds = (uint32_t)ChainLds<D, TI>::bytes((a.N + 15) & ~15);
 #define SLOT_CF(RR) if (a.N <= 64 * RR) { \
         if (a.cslog) slothost::launch((chain_fwd<D, RR, TI, true>), grid, block, lds, st, a); \
@@ -3014,20 +3049,58 @@ static int fwd_chunks(int64_t B, int64_t T, int64_t H, int64_t N, int64_t G, int
     return n;
 }
 
+// Chains that chain_fwd holds at once: workgroups per CU by their LDS records, on 256 CUs.
+static int64_t fwd_round(int64_t N, int64_t D, int dtype) {
+    const int NP = (int)((N + 15) & ~15ll);
+    const size_t lds = D == 128 ? (dtype == SLOTSCAN_BF16 ? ChainLds<128, bf16_t>::bytes(NP) : ChainLds<128, float>::bytes(NP))
+                                : (dtype == SLOTSCAN_BF16 ? ChainLds<64, bf16_t>::bytes(NP) : ChainLds<64, float>::bytes(NP));
+    return 256 * std::max<int64_t>(1, 163840 / (int64_t)lds);
+}
+
 // Batch rows of one group where a one-chunk forward runs as a pipeline over groups of whole batch rows (B: no
 // groups).  chain_fwd's LDS records let a round of its workgroups hold only so many chains; beyond that the rounds
 // follow each other anyway, so the replay of one group runs beside the chains of the next.  A group is at least
 // one round, and enough rounds of a short scan that its chains take about the 100 us that hide its launches.
 static int64_t fwd_group(int64_t B, int64_t T, int64_t H, int64_t N, int64_t D, int dtype) {
-    const int64_t NP = (N + 15) & ~15ll;
-    const size_t lds = D == 128 ? (dtype == SLOTSCAN_BF16 ? ChainLds<128, bf16_t>::bytes((int)NP) : ChainLds<128, float>::bytes((int)NP))
-                                : (dtype == SLOTSCAN_BF16 ? ChainLds<64, bf16_t>::bytes((int)NP) : ChainLds<64, float>::bytes((int)NP));
-    const int64_t round = 256 * std::max<int64_t>(1, 163840 / (int64_t)lds);
-    const int64_t chains = round * std::max<int64_t>(1, 192 / T);
+    const int64_t chains = fwd_round(N, D, dtype) * std::max<int64_t>(1, 192 / T);
     if (B * H <= chains) return B;
     int64_t g = std::max<int64_t>(1, chains / H);
     g = std::max<int64_t>(g, (B + FWD_MAX_CHUNKS - 2) / (FWD_MAX_CHUNKS - 1));
     return std::min<int64_t>(B, g);
+}
+
+// Whether the keys stay in registers (chain_fwd_reg) in chunks of `Tc` steps.  With fp32 snapshots, D 128 and N > 96 it is
+// the better one for more chains than a round of chain_fwd at any length (at the kernel).  Elsewhere a step of
+// chain_fwd takes a third of the time, but a round of it is as many chains or half as many (over 80 KB of records),
+// and its start and end, the state's way through LDS, take about 13 us at N 192, D 128 against 5: where the chains
+// need more rounds and the scan is short, the register chain is through sooner.  Forward without logs, G 8, us with
+// chain_fwd / chain_fwd_reg (rounds of each), D 128 and bf16 tokens unless noted:
+//   bf16 copies  N 192, 1,024 chains (4, 2): T 16 113 / 91, T 64 315 / 287, T 96 420 / 452;  512 (2, 1): T 32 97 / 82, T 96
+//                230 / 216, T 128 258 / 283;  768 (3, 2): T 64 241 / 242;  N 128, 1,024: T 16 87 / 82, T 48 187 / 193
+//   fp32 copies  D 64, N 192, fp32 tokens, 512 (2, 1): T 64 147 / 125, T 128 236 / 237;  1,024 (4, 2): T 96 357 / 350, T 128
+//                402 / 458;  bf16 tokens, 1,024 (2, 2): T 16 76 / 70, T 32 129 / 127, T 64 232 / 237;  N 96, fp32 tokens,
+//                1,024 (4, 2): T 64 273 / 270, T 96 372 / 396
+//   codes        N 192, 1,024 (4, 2): T 4 103 / 88, T 16 132 / 117, T 48 227 / 235;  N 128: T 8 84 / 79, T 32 141 / 152
+static bool fwd_chain_reg(int mode, int bits, int64_t chains, int64_t Tc, int64_t N, int64_t D, int dtype) {
+    if (N <= 64) return false;                           // its rounds are never the larger ones
+    const bool f32 = mode == FE_F32, mem = mode == FE_MEM && !bits;
+    if (f32 && D == 128 && N > 96 && chains > 256) return true;
+    const int64_t cap = fwd_round(N, D, dtype), rcap = D == 64 && N <= 96 ? 1024 : 512;     // chains at once
+    const int64_t rn = (chains + cap - 1) / cap, rr = (chains + rcap - 1) / rcap;           // rounds
+    const bool wide = N > 128;                           // chain_fwd: three rows a lane
+    const bool full = 4 * chains >= 3 * cap * rn;        // the last round is not a small one
+    const bool twice = full && rn >= 2 * rr, once = twice && rr == 1;
+    int64_t lim = 0;
+    if (rn > rr) {
+        if (f32) lim = wide ? (once ? 128 : 96) : once ? 96 : twice ? 64 : 32;
+        else if (mem) lim = !wide ? (twice ? 16 : 8) : once && D == 128 ? 96 : twice ? (rr <= 2 ? 64 : 48) : D == 128 ? 64 : 16;
+        else lim = wide ? 16 : 8;
+    } else if (full && wide) {                           // as many rounds: only the start is longer
+        lim = f32 ? (Tc > 8 || rn > 4 ? 32 : 0) : rn == 1 ? 0 : mem ? 4 : 8;
+    } else if (full && f32 && D == 128 && rn > 1) {
+        lim = 4;
+    }
+    return Tc <= lim;
 }
 
 static int check_q(int bits, int64_t group, int64_t D, bool codes) {
@@ -3049,7 +3122,7 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
     if (int r = check_common(B, T, H, N, D, G, dtype)) return r;
     const int mode = o.mode;
     int64_t cb[FWD_MAX_CHUNKS + 1] = {0, T};
-        const int nch = o.one ? 1 : fwd_chunks(B, T, H, N, G, cb);
+    const int nch = o.one ? 1 : fwd_chunks(B, T, H, N, G, cb);
     if (!k || !q || !v || !gate || !fr || !temp || !am || !kfin || !vfin || !ofin ||
         (mode == FE_F32 && (!o.kbuf || !o.vbuf)) ||
         (mode == FE_MEM && (!o.kbm || !o.vbm || !o.kinvm || !o.validm)) ||
@@ -3067,11 +3140,11 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
     hipStream_t st = (hipStream_t)stream;
     const int NB = (int)((T + G - 1) / G);
     const bool f32 = mode == FE_F32;
-    // the register-resident chain: built for D = 128 and more than 96 rows, where chain_fwd's records leave room for
-    // one workgroup on each of the 256 CUs
-    const bool reg = f32 && D == 128 && N > 96 && B * H > 256;
+    const bool reg = fwd_chain_reg(mode, o.bits, B * H, nch > 1 ? fwd_chunk_len(T, G) : T, N, D, dtype);
+    const bool keys = reg && (f32 || (mode == FE_MEM && !o.bits));       // the chain emits the keys' copies itself
     ChainFwdArgs ca{q, k, gate, fr, temp, k0, o0, am, oold, cslog, kfin, ofin, (int)T, (int)H, (int)N, eps,
-                    fr_per_token ? 1 : 0, occ_bin ? 1 : 0, 0, (int)T, o.kbuf, kold, (int)G, NB, (int)H, (int)H, 0};
+                    fr_per_token ? 1 : 0, occ_bin ? 1 : 0, 0, (int)T, o.kbuf, keys ? o.kbm : nullptr, o.kinvm, o.validm, kold,
+                    (int)G, NB, (int)H, (int)H, 0};
     RowsFwdArgs ra{k, v, gate, am, k0, v0, nullptr, vfin, kold, vold, (int)T, (int)H, (int)N, (int)G, NB, 0, (int)T,
                    (int)H, (int)H, (int)H, (int)H, 0, o.kbuf, o.vbuf, o.kbm, o.vbm, o.kinvm, o.validm,
                    o.kcode, o.kscale, o.vcode, o.vscale, o.bits, o.group};
@@ -3123,7 +3196,7 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
         const bool inner_end = ca.te < T;
         if (ch > 0) {
             ca.o0 = ofin;
-            ca.k0 = reg ? o.kbuf + (size_t)(ca.ts / G) * H * N * D : kfin;
+            ca.k0 = reg && f32 ? o.kbuf + (size_t)(ca.ts / G) * H * N * D : kfin;
             if (f32) {
                 ca.k0bs = NB * (int)H;
                 ca.skip0 = 1;
@@ -3164,7 +3237,8 @@ static int scan_fwd(const void* k, const void* q, const void* v, int dtype,
         }
         {
             slothost::Scope sc(SLOTSCAN_K_ROWS_FWD, rs);
-#define SLOT_RF(DD, TT) { if (mode == FE_MEM) slothost::launch((rows_fwd<DD, TT, RF_MEM>), grid, block, 0, rs, ra); \
+#define SLOT_RF(DD, TT) { if (mode == FE_MEM && keys) slothost::launch((rows_fwd<DD, TT, RF_MEMV>), grid, block, 0, rs, ra); \
+                          else if (mode == FE_MEM) slothost::launch((rows_fwd<DD, TT, RF_MEM>), grid, block, 0, rs, ra); \
                           else if (mode == FE_CODES) slothost::launch((rows_fwd<DD, TT, RF_CODES>), grid, block, 0, rs, ra); \
                           else if (reg) slothost::launch((rows_fwd<DD, TT, RF_F32V>), grid, block, 0, rs, ra); \
                           else slothost::launch((rows_fwd<DD, TT, RF_F32>), grid, block, 0, rs, ra); }

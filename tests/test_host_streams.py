@@ -7,7 +7,10 @@ import sys
 
 import pytest
 
+import torch
+
 import slotscan_lib as L
+from test_gpu_scan_reg import CASES as REG_CASES
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 
@@ -20,6 +23,17 @@ stub.stub_capture.argtypes = [ctypes.c_void_p, ctypes.c_uint64]
 lib = ctypes.CDLL(sys.argv[2])
 vp, i64, i32, f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
 lib.slotscan_fwd.argtypes = [vp, vp, vp, i32, vp, vp, i32, vp] + [i64] * 6 + [f32, i32] + [vp] * 14
+lib.slotscan_fwd_memq.argtypes = [vp, vp, vp, i32, vp, vp, i32, vp] + [i64] * 6 + [f32, i32, i32, i64] + [vp] * 17
+lib.slotscan_fwd_codes.argtypes = [vp, vp, vp, i32, vp, vp, i32, vp] + [i64] * 6 + [f32, i32, i32, i64] + [vp] * 13
+def call_mode(mode, bf16, B, T, H, N, D, G):
+    p = 1 << 20
+    a = (p, p, p, bf16, p, p, 1, p, B, T, H, N, D, G, 1e-4, 1)
+    if mode == "f32":
+        return lib.slotscan_fwd(*a, None, None, None, p, p, p, None, None, None, None, p, p, p, None)
+    if mode == "codes":
+        return lib.slotscan_fwd_codes(*a, 8, D, None, None, None, p, p, p, p, p, p, p, p, p, None)
+    return lib.slotscan_fwd_memq(*a, 3 if mode == "memq" else 0, 16, None, None, None, p, p, p, p, p, None, None, None, None,
+                                 p, p, p, p, None)
 def call(thread, stream, B=8, T=1024, H=6, N=192, D=128, G=8):
     stub.stub_thread(thread)
     p = 1 << 20
@@ -126,3 +140,38 @@ print(json.dumps(log()))
     assert sum(op[1] == "launch" for op in log) == n + 1 and side
     joined = [k for k, op in enumerate(log) if op[1] == "record" and op[3] == log[side[0]][3] and k > side[-1]]
     assert joined and any(op[1] == "wait" and op[2] == "0x100" and op[3] == log[joined[0]][2] for op in log[joined[0]:])
+
+
+def _chains(stub, shapes):
+    """For each (mode, bf16, B, T, H, N, D, G): the set of chain kernels that the forward launches."""
+    logs = _run(stub, f"""
+out = []
+for c in {shapes!r}:
+    stub.stub_reset()
+    assert call_mode(*c) == 0, c
+    out.append([op[2] for op in log() if op[1] == "launch"])
+print(json.dumps(out))
+""")
+    return [{"reg" if "chain_fwd_reg" in n else "lds" for n in names if "chain_fwd" in n} for names in logs]
+
+
+def test_register_chain_cases_take_it(stub):
+    """The cases whose outputs test_gpu_scan_reg.py compares do run the register chain, and a few of their rows the other."""
+    many = [(c[0], int(c[7] == torch.bfloat16), c[1], *c[2:7]) for c in REG_CASES]
+    assert _chains(stub, many) == [{"reg"}] * len(many)
+    assert _chains(stub, [(*c[:2], 3, *c[3:]) for c in many]) == [{"lds"}] * len(many)
+
+
+# mode, bf16 tokens, chains (H 8), N, D, the longest scan that keeps its keys in registers
+@pytest.mark.parametrize("mode,bf16,chains,N,D,longest", [
+    ("f32", 1, 256, 192, 128, 0), ("f32", 1, 264, 192, 128, 4096), ("f32", 1, 4096, 96, 128, 4), ("f32", 0, 1024, 96, 128, 64),
+    ("f32", 0, 512, 192, 64, 128), ("f32", 0, 1024, 192, 64, 96), ("f32", 1, 1024, 96, 64, 32), ("f32", 1, 4096, 64, 128, 0),
+    ("mem", 1, 256, 192, 128, 0), ("mem", 1, 264, 192, 128, 64), ("mem", 1, 512, 192, 128, 96), ("mem", 1, 4096, 192, 128, 48),
+    ("mem", 1, 1024, 128, 128, 16), ("mem", 1, 768, 128, 128, 8), ("mem", 0, 768, 192, 64, 16), ("mem", 1, 1024, 96, 64, 8),
+    ("memq", 1, 1024, 192, 128, 16), ("codes", 1, 1024, 192, 128, 16), ("codes", 1, 1024, 128, 128, 8), ("codes", 1, 4096, 96, 128, 0),
+])
+def test_register_chain_rule(stub, mode, bf16, chains, N, D, longest):
+    """Both sides of the rule's line."""
+    c = lambda T: (mode, bf16, chains // 8, T, 8, N, D, 8)
+    sides = ([(c(longest), {"reg"})] if longest else []) + ([(c(longest + 1), {"lds"})] if longest < 4096 else [])
+    assert _chains(stub, [s for s, _ in sides]) == [want for _, want in sides]
