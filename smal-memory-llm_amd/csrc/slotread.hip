@@ -1101,6 +1101,8 @@ template <int L> __device__ __forceinline__ float prep_sum(float v) {       // o
     if constexpr (L == 16) v += dppf<SLOT_DPP_MIR>(v);
     return v;
 }
+// max(|q|, 1e-6) rounded to bf16, as in q's dtype; a NaN stays one (fmaxf would drop it)
+__device__ __forceinline__ float prep_norm(float nrm) { return bf16_round(nrm < 1e-6f ? 1e-6f : nrm); }
 __device__ __forceinline__ void prep_unpack(uint4 r, float* x) {
     const uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
@@ -1121,8 +1123,7 @@ __global__ __launch_bounds__(PREP_THREADS) void read_prep(PrepArgs a) {
         prep_unpack(*reinterpret_cast<const uint4*>(a.q + at), x);
 #pragma unroll
         for (int e = 0; e < 8; e++) qq = fmaf(x[e], x[e], qq);
-        // the norm is rounded to bf16 before the division, as in q's dtype
-        const float nb = bf16_round(fmaxf(__fsqrt_rn(prep_sum<L>(qq)), 1e-6f));
+        const float nb = prep_norm(__fsqrt_rn(prep_sum<L>(qq)));
         uint4 r;
         r.x = pack_bf16x2(x[0] / nb, x[1] / nb);
         r.y = pack_bf16x2(x[2] / nb, x[3] / nb);
@@ -1156,7 +1157,7 @@ __global__ __launch_bounds__(PREP_THREADS) void read_prep_bwd(PrepArgs a) {
         for (int e = 0; e < 8; e++) { qq = fmaf(x[e], x[e], qq); dot = fmaf(x[e], d[e], dot); }
         const float nrm = __fsqrt_rn(prep_sum<L>(qq));
         dot = prep_sum<L>(dot);
-        const float nb = bf16_round(fmaxf(nrm, 1e-6f));
+        const float nb = prep_norm(nrm);
         const float co = nrm >= 1e-6f ? dot / nb / nb / nrm : 0.f;
         float y[8];
 #pragma unroll

@@ -70,3 +70,28 @@ def test_prep_takes_views_and_leaves_broadcasts_to_torch():
         torch.testing.assert_close(qn.float(), base[0].float(), rtol=2.0 ** -7, atol=1e-30)
     qn, sc = RH._prep(q, lr, s[:, :, :1, :1], 2.0)
     torch.testing.assert_close(sc[:, :, 0, 0], base[1][:, :, 0, 0], rtol=2e-6, atol=0)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_prep_passes_nan_and_infinity_on(D):
+    """A NaN in a query makes its norm NaN, and with it the whole unit query and its gradient; an infinity leaves 0 and NaN.
+    As the torch expressions; the other queries are untouched."""
+    q, s, dqn, dsc = (x.cuda() for x in _inputs(2, 5, 3, 2, D, 11))
+    lr = torch.tensor(0.3, device="cuda")
+    bad = q.clone()
+    bad[0, 1, 2, 0, 5] = float("nan")
+    bad[1, 3, 0, 1, D - 1] = float("inf")
+
+    def run(x, prep):
+        x = x.clone().requires_grad_()
+        qn, sc = prep(x)
+        return qn.detach(), sc, torch.autograd.grad([qn], [x], [dqn])[0]
+
+    a, b = run(bad, lambda x: RH._prep(x, lr, s, 2.0)), run(q, lambda x: RH._prep(x, lr, s, 2.0))
+    t = run(bad, lambda x: (x / x.float().norm(dim=-1, keepdim=True).clamp_min(1e-6).to(x.dtype), None))
+    assert a[0][0, 1, 2, 0].isnan().all() and a[2][0, 1, 2, 0].isnan().all()
+    for i in (0, 2):
+        assert torch.equal(a[i].isnan(), t[i].isnan())
+    same = torch.ones(q.shape[:-1], dtype=torch.bool, device="cuda")
+    same[0, 1, 2, 0] = same[1, 3, 0, 1] = False
+    assert torch.equal(a[0][same], b[0][same]) and torch.equal(a[1], b[1]) and torch.equal(a[2][same], b[2][same])
