@@ -132,15 +132,22 @@ class _PrepHip(torch.autograd.Function):
         return dq, ds, dl.reshape(lshape), None
 
 
+def _prep_fused(q, log_rsel, s, rsharp):
+    """Whether _prep's call takes the kernels: what they read directly, and nothing that the torch expressions refuse (a
+    log_rsel of more dimensions than the multiplier)."""
+    return (q.is_cuda and q.dtype == torch.bfloat16 and q.shape[-1] in _SUPPORTED_D and q.numel() > 0
+            and torch.is_tensor(log_rsel) and log_rsel.numel() == 1 and log_rsel.dim() <= 4
+            and log_rsel.device == q.device and log_rsel.is_floating_point()
+            and (rsharp is None or isinstance(rsharp, (int, float)))
+            and (s is None or (s.shape == q.shape[:-1] and s.device == q.device and s.is_floating_point())))
+
+
 def _prep(q, log_rsel, s, rsharp):
     """(unit queries, multiplier) of memlm_sh.py:379-393.  bf16 queries with one log_rsel and an s of their own shape --
     what the layer passes -- take one kernel each way (one pass over q instead of seven; measured there); other
     dtypes, and a log_rsel or s that broadcasts, the same expressions in torch."""
     B, T, H, NQ, D = q.shape
-    if (q.is_cuda and q.dtype == torch.bfloat16 and D in _SUPPORTED_D and q.numel() and torch.is_tensor(log_rsel)
-            and log_rsel.numel() == 1 and log_rsel.device == q.device and log_rsel.is_floating_point()
-            and (rsharp is None or isinstance(rsharp, (int, float)))
-            and (s is None or (s.shape == q.shape[:-1] and s.device == q.device and s.is_floating_point()))):
+    if _prep_fused(q, log_rsel, s, rsharp):
         return _PrepHip.apply(q, None if s is None else s.float(), log_rsel.float(),
                               0.0 if s is None or not rsharp else float(rsharp))
     qn = q / q.float().norm(dim=-1, keepdim=True).clamp_min(1e-6).to(q.dtype)

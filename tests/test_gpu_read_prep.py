@@ -95,3 +95,13 @@ def test_prep_passes_nan_and_infinity_on(D):
     same = torch.ones(q.shape[:-1], dtype=torch.bool, device="cuda")
     same[0, 1, 2, 0] = same[1, 3, 0, 1] = False
     assert torch.equal(a[0][same], b[0][same]) and torch.equal(a[1], b[1]) and torch.equal(a[2][same], b[2][same])
+
+
+def test_prep_refuses_a_log_rsel_that_does_not_expand():
+    """One value in more dimensions than the multiplier (B, T, H, NQ) has was never accepted."""
+    q, s, _, _ = (x.cuda() for x in _inputs(2, 3, 2, 1, 64, 5))
+    base = RH._prep(q, torch.tensor(0.3, device="cuda"), s, 2.0)
+    for n in range(5):
+        assert all(torch.equal(a, b) for a, b in zip(RH._prep(q, torch.full((1,) * n, 0.3, device="cuda"), s, 2.0), base))
+    with pytest.raises(RuntimeError):
+        RH._prep(q, torch.full((1,) * 5, 0.3, device="cuda"), s, 2.0)
