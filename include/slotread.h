@@ -49,7 +49,8 @@ int slotread_bwd(const void* q, const void* kbuf, const void* vbuf, const float*
 
 /* The read's query preparation in one pass (memlm_sh.py:379-393): qn = q / max(|q|, 1e-6) with the norm rounded to
  * bf16, scale = exp(log_rsel) exp(sharp tanh(s / sharp)) (sharp 0: exp(s); s NULL: exp(log_rsel)).
- *   q, qn (rows, D) bf16, 16-byte aligned, D 64 or 128;  s, scale (rows) fp32;  log_rsel one fp32.
+ *   q, qn (rows, D) bf16, 16-byte aligned, D 64 or 128, at most 8 (2^32 - 256) elements;  s, scale (rows) fp32;
+ *   log_rsel one fp32.
  * Backward: dqn (rows, D) bf16 and dscale (rows) fp32 in; dq (rows, D) bf16, ds (rows, with s), dlog_rsel (one) out;
  * workspace slotread_prep_workspace(rows, D) bytes. */
 size_t slotread_prep_workspace(int64_t rows, int64_t D);

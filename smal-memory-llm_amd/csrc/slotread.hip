@@ -1317,7 +1317,8 @@ extern "C" int slotread_bwd(const void* q, const void* kbuf, const void* vbuf, c
 
 static int check_prep(int64_t rows, int64_t D) {
     if (rows < 1 || (D != 64 && D != 128)) return fail(SLOTSCAN_ERR_SHAPE, "slotread_prep: rows >= 1, D 64 or 128");
-    if (rows > 0x7fffffffLL * 16) return fail(SLOTSCAN_ERR_SHAPE, "slotread_prep: too many rows");
+    // a launch is at most 2^32 - 1 lanes, D / 8 of them a row
+    if (rows > (0xffffff00LL / (D / 8))) return fail(SLOTSCAN_ERR_SHAPE, "slotread_prep: more than 2^32 - 256 lanes of 8 elements");
     return 0;
 }
 

@@ -132,10 +132,14 @@ class _PrepHip(torch.autograd.Function):
         return dq, ds, dl.reshape(lshape), None
 
 
+# slotread_prep_*: at most 2^32 lanes of 8 elements in one launch (68 GB of queries)
+_PREP_MAX = 8 * (2 ** 32 - 256)
+
+
 def _prep_fused(q, log_rsel, s, rsharp):
     """Whether _prep's call takes the kernels: what they read directly, and nothing that the torch expressions refuse (a
     log_rsel of more dimensions than the multiplier)."""
-    return (q.is_cuda and q.dtype == torch.bfloat16 and q.shape[-1] in _SUPPORTED_D and q.numel() > 0
+    return (q.is_cuda and q.dtype == torch.bfloat16 and q.shape[-1] in _SUPPORTED_D and 0 < q.numel() <= _PREP_MAX
             and torch.is_tensor(log_rsel) and log_rsel.numel() == 1 and log_rsel.dim() <= 4
             and log_rsel.device == q.device and log_rsel.is_floating_point()
             and (rsharp is None or isinstance(rsharp, (int, float)))

@@ -190,6 +190,25 @@ def test_proj_bwd_validation_rejects_before_launch(M, N, K, code):
     assert ws >= 2048 * 768 * 2 + 2048 * 768 * 4 and (ws - ((2048 * 768 * 2 + 255) & ~255)) % (2048 * 768 * 4) == 0
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_prep_refuses_more_rows_than_a_launch_holds(D):
+    """slotread_prep_* run D / 8 lanes a row in one launch of fewer than 2^32: more rows are refused before any GPU call,
+    and the Python entry points leave them to torch."""
+    import types
+
+    import slotread_hip as RH
+    p, most = ctypes.c_void_p(1 << 20), (2 ** 32 - 256) // (D // 8)
+    assert most * D == RH._PREP_MAX
+    for rows in (most + 1, 2 ** 40):
+        assert L.lib().slotread_prep_fwd(p, p, p, 2.0, rows, D, p, p, None) == 1
+        assert L.lib().slotread_prep_bwd(p, p, p, p, p, 2.0, rows, D, p, p, p, p, None) == 1
+    import torch
+    q = lambda rows: types.SimpleNamespace(is_cuda=True, dtype=torch.bfloat16, shape=(1, rows, 1, 1, D),
+                                           device=torch.device("cpu"), numel=lambda: rows * D)
+    lr = torch.zeros(())
+    assert RH._prep_fused(q(most), lr, None, None) and not RH._prep_fused(q(most + 1), lr, None, None)
+
+
 @pytest.mark.parametrize("which", ["out", "dq", "dk", "dv"])
 def test_window_refuses_8_byte_aligned_outputs(which):
     """win_fwd / win_bwd write out, dq, dk and dv as 16-byte row pieces: an 8-byte-aligned output pointer is
