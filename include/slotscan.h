@@ -70,11 +70,10 @@ int slotscan_fwd(const void* k, const void* q, const void* v, int dtype,
 size_t slotscan_bwd_workspace(int64_t B, int64_t T, int64_t H, int64_t N);
 
 /* Which backward kernels slotscan_bwd (mem = 0) or slotscan_bwd_mem (mem = 1) runs for a shape, as a bit
- * set; no GPU work.  SLOTSCAN_PLAN_ROWS_UNTRACKED: the row kernel's variant with explicitly counted
- * loads, used when G == 8, T % 16 == 0 (D == 128 for mem) and a batch row's snapshot gradients span at
- * most 4 GiB (its loads use 32-bit offsets).  SLOTSCAN_PLAN_ROWS_UNTRACKED_PART: the same variant with a padded
- * last chunk (G == 8, T % 16 != 0) or one snapshot per 16 steps (G == 16).  Otherwise the compiler-tracked
- * variant runs.  Returns -1 for
+ * set; no GPU work.  SLOTSCAN_PLAN_ROWS_UNTRACKED: the row kernel's variant with explicitly counted loads, used when
+ * G is 8 or 16 (D == 128 for mem) and a batch row's snapshot gradients span at most 4 GiB (its loads use 32-bit
+ * offsets); otherwise the compiler-tracked variant runs.  SLOTSCAN_PLAN_ROWS_UNTRACKED_PART, only beside it: that
+ * variant with a padded last chunk (T % 16 != 0) or one snapshot per 16 steps (G == 16).  Returns -1 for
  * an invalid shape.  No counterpart in the reference (whose backward has one kernel per direction): it lets
  * a caller, and the CPU tests, see the choice the library makes. */
 #define SLOTSCAN_PLAN_ROWS_UNTRACKED 1

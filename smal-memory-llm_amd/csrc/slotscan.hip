@@ -3337,7 +3337,7 @@ extern "C" int slotscan_bwd_plan(int64_t T, int64_t H, int64_t N, int64_t D, int
         return -1;
     }
     if (!rows_bwd_untracked(T, H, N, D, G, mem != 0)) return 0;
-    return G == 8 && T % 16 == 0 ? SLOTSCAN_PLAN_ROWS_UNTRACKED : SLOTSCAN_PLAN_ROWS_UNTRACKED_PART;
+    return SLOTSCAN_PLAN_ROWS_UNTRACKED | (G == 8 && T % 16 == 0 ? 0 : SLOTSCAN_PLAN_ROWS_UNTRACKED_PART);
 }
 
 extern "C" size_t slotscan_bwd_workspace(int64_t B, int64_t T, int64_t H, int64_t N) {

@@ -102,23 +102,38 @@ def test_dtype_codes():
         L.dtype_code(torch.float16)
 
 
-@pytest.mark.parametrize("T,H,N,D,G,mem,untracked", [
-    (1024, 6, 192, 128, 8, 0, True),        # config 2
-    (1024, 6, 192, 128, 8, 1, True),        # config 2, fused epilogue
-    (1024, 6, 192, 64, 8, 1, False),        # the fused contract's untracked kernel is built for D = 128
-    (1000, 6, 192, 128, 8, 0, False),       # T % 16 != 0
-    (1024, 6, 192, 128, 7, 0, False),       # G != 8
-    (58240, 6, 192, 128, 8, 0, True),       # NB * H * N * D * 4 = 4,293,918,720 B: just fits 32 bits
-    (58256, 6, 192, 128, 8, 0, False),      # 4,295,098,368 B: past 2^32, the tracked kernel runs
-    (58256, 6, 192, 128, 8, 1, True),       # bf16 gradients: half the bytes
-    (116512, 6, 192, 128, 8, 1, False),
+# bytes of a batch row's snapshot gradients: ceil(T / G) H N D, times 4 (mem: bf16, times 2); 2^32 - 1 is the most
+@pytest.mark.parametrize("T,H,N,D,G,mem,untracked,part", [
+    (1024, 6, 192, 128, 8, 0, True, False),         # config 2
+    (1024, 6, 192, 128, 8, 1, True, False),         # config 2, fused epilogue
+    (1024, 6, 192, 64, 8, 1, False, False),         # the fused contract's untracked kernel is built for D = 128
+    (1000, 6, 192, 128, 8, 0, True, True),          # T % 16 != 0: a padded last chunk
+    (1000, 6, 192, 128, 8, 1, True, True),
+    (1024, 6, 192, 128, 16, 0, True, True),         # G = 16: one snapshot per chunk
+    (1, 1, 1, 64, 16, 0, True, True),
+    (1024, 6, 192, 128, 7, 0, False, False),        # any other G
+    (1024, 6, 192, 128, 4, 1, False, False),
+    (58240, 6, 192, 128, 8, 0, True, False),        # NB * H * N * D * 4 = 4,293,918,720 B: just fits 32 bits
+    (58256, 6, 192, 128, 8, 0, False, False),       # 4,295,098,368 B: past 2^32, the tracked kernel runs
+    (58256, 6, 192, 128, 8, 1, True, False),        # bf16 gradients: half the bytes
+    (116512, 6, 192, 128, 8, 1, False, False),
+    (58241, 6, 192, 128, 8, 0, True, True),         # ragged: 7,281 blocks are 4,294,508,544 B, 7,282 are 4,295,098,368 B
+    (58249, 6, 192, 128, 8, 0, False, False),
+    (116504, 6, 192, 128, 8, 1, True, True),        # 14,563 blocks, 4,294,803,456 B; one step more is a block more
+    (116505, 6, 192, 128, 8, 1, False, False),
+    (116496, 6, 192, 128, 16, 0, True, True),       # the same blocks at G = 16
+    (116497, 6, 192, 128, 16, 0, False, False),
+    (233008, 6, 192, 128, 16, 1, True, True),
+    (233009, 6, 192, 128, 16, 1, False, False),
 ])
-def test_bwd_plan_untracked_rows_kernel_guard(T, H, N, D, G, mem, untracked):
-    """The untracked G = 8 row kernel forms a batch row's snapshot-gradient offsets in 32 bits: the library
-    uses it only where they fit (slotscan_bwd_plan exposes the choice; no GPU work)."""
+def test_bwd_plan_untracked_rows_kernel_guard(T, H, N, D, G, mem, untracked, part):
+    """The counted-load row kernel (G = 8, and G = 16) forms a batch row's snapshot-gradient offsets in 32 bits: the library
+    uses it only where they fit (slotscan_bwd_plan exposes the choice; no GPU work).  Bit 1 says that it runs, bit 2
+    that it runs with a padded last chunk or one snapshot per chunk."""
     plan = L.lib().slotscan_bwd_plan(T, H, N, D, G, mem)
+    assert untracked == ((T + G - 1) // G * H * N * D * (2 if mem else 4) < 2 ** 32 and G in (8, 16) and (D == 128 or not mem))
     assert plan >= 0
-    assert bool(plan & 1) == untracked
+    assert bool(plan & 1) == untracked and bool(plan & 2) == part
     assert L.lib().slotscan_bwd_plan(0, H, N, D, G, mem) == -1
 
 
