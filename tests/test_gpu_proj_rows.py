@@ -1,5 +1,6 @@
-"""The projection's few-row kernel and both sides of the rule that chooses it, forward (with and without the residual)
-and the backward's dRD, against float64.  Guard rows behind the output stay untouched."""
+"""The projection's few-row kernel and both sides of the rule that chooses it, forward, with and without the residual, and
+the backward's products at the same row counts, which the tile kernels form, against float64.  Guard rows behind the
+output stay untouched.  test_host_streams.py checks on the CPU which kernel each case here runs."""
 import pytest
 import torch
 
@@ -16,11 +17,17 @@ def _bound(ref, mag, K):
     return 2.0 ** -8 * 1.02 * ref.abs() + K * 2.0 ** -24 * mag
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (1, 256, 32), (15, 256, 64), (16, 256, 224), (17, 512, 256), (32, 256, 1536), (33, 256, 288), (64, 2048, 1536),
-    (65, 512, 512), (128, 1024, 96), (256, 2048, 64), (257, 2048, 64), (300, 2048, 96), (2048, 256, 64),
-    (2049, 256, 64),
-])
+# (M, N, K), whether the few-row kernel runs
+FORWARD = [
+    ((1, 256, 32), True), ((15, 256, 64), True), ((16, 256, 224), True), ((17, 512, 256), True), ((32, 256, 1536), True),
+    ((33, 256, 288), True), ((64, 2048, 1536), True), ((65, 512, 512), True), ((128, 1024, 96), True),
+    ((256, 2048, 64), True), ((257, 2048, 64), False), ((300, 2048, 96), False), ((2048, 256, 64), True),
+    ((2049, 256, 64), False),
+]
+BACKWARD = [(5, 256, 256), (40, 512, 1024), (70, 2048, 256), (700, 256, 1024)]
+
+
+@pytest.mark.parametrize("M,N,K", [s for s, _ in FORWARD])
 @pytest.mark.parametrize("res", [True, False])
 def test_proj_rows_matches_float64(M, N, K, res):
     gen = torch.Generator().manual_seed(M + N + K)
@@ -39,8 +46,8 @@ def test_proj_rows_matches_float64(M, N, K, res):
     assert (out[M:] == 7.0).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(5, 256, 256), (40, 512, 1024), (70, 2048, 256), (700, 256, 1024)])
-def test_proj_rows_backward(M, N, K):
+@pytest.mark.parametrize("M,N,K", BACKWARD)
+def test_few_rows_backward(M, N, K):
     gen = torch.Generator().manual_seed(3 * M + K)
     g = torch.randn(M, N, generator=gen).to(torch.bfloat16).cuda()
     x = torch.randn(M, K, generator=gen).to(torch.bfloat16).cuda()

@@ -97,6 +97,29 @@ def test_prep_passes_nan_and_infinity_on(D):
     assert torch.equal(a[0][same], b[0][same]) and torch.equal(a[1], b[1]) and torch.equal(a[2][same], b[2][same])
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_prep_gradient_error_is_no_larger_than_the_torch_expressions(D):
+    """dq is formed in fp32 and rounded to bf16 once, where the torch expressions round every intermediate result: the two
+    differ (2.9e-3, 2-norm), and the kernel's is the one closer to float64 (2.3e-3 against 2.9e-3)."""
+    gen = torch.Generator().manual_seed(9)
+    q = torch.randn(4, 256, 6, 2, D, generator=gen).to(torch.bfloat16).cuda()
+    d = torch.randn(q.shape, generator=gen).to(torch.bfloat16).cuda()
+    lr = torch.tensor(0.0, device="cuda")
+    norm = lambda x: x / x.float().norm(dim=-1, keepdim=True).clamp_min(1e-6).to(x.dtype)
+    exact = lambda x: x / x.norm(dim=-1, keepdim=True).clamp_min(1e-6)
+
+    def grad(x, f):
+        x = x.clone().requires_grad_()
+        return torch.autograd.grad(f(x), x, d.to(x.dtype))[0].double()
+
+    ref = grad(q.double(), exact)
+    err = lambda f: ((grad(q, f) - ref).norm() / ref.norm()).item()
+    kern, expr = err(lambda x: RH._prep(x, lr, None, None)[0]), err(norm)
+    print(f"dq against float64: kernel {kern:.2e}, torch expressions {expr:.2e}")
+    # the norm's rounding, common to a query, and the result's: each uniform within 2^-8 of the value at most
+    assert kern <= expr and kern <= 2 * 2.0 ** -8 / 3 ** 0.5
+
+
 def test_prep_refuses_a_log_rsel_that_does_not_expand():
     """One value in more dimensions than the multiplier (B, T, H, NQ) has was never accepted."""
     q, s, _, _ = (x.cuda() for x in _inputs(2, 3, 2, 1, 64, 5))

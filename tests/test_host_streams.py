@@ -10,6 +10,8 @@ import pytest
 import torch
 
 import slotscan_lib as L
+from test_gpu_proj_rows import BACKWARD, FORWARD
+from test_gpu_scan_groups import GROUPS
 from test_gpu_scan_reg import CASES as REG_CASES
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -34,6 +36,8 @@ def call_mode(mode, bf16, B, T, H, N, D, G):
         return lib.slotscan_fwd_codes(*a, 8, D, None, None, None, p, p, p, p, p, p, p, p, p, None)
     return lib.slotscan_fwd_memq(*a, 3 if mode == "memq" else 0, 16, None, None, None, p, p, p, p, p, None, None, None, None,
                                  p, p, p, p, None)
+lib.slotproj_fwd.argtypes = [vp, vp, vp, i64, i64, i64, vp, vp]
+lib.slotproj_bwd.argtypes = [vp, vp, vp, i64, i64, i64, vp, vp, vp, vp]
 def call(thread, stream, B=8, T=1024, H=6, N=192, D=128, G=8):
     stub.stub_thread(thread)
     p = 1 << 20
@@ -175,3 +179,46 @@ def test_register_chain_rule(stub, mode, bf16, chains, N, D, longest):
     c = lambda T: (mode, bf16, chains // 8, T, 8, N, D, 8)
     sides = ([(c(longest), {"reg"})] if longest else []) + ([(c(longest + 1), {"lds"})] if longest < 4096 else [])
     assert _chains(stub, [s for s, _ in sides]) == [want for _, want in sides]
+
+
+def test_batch_group_cases_run_in_groups(stub):
+    """The cases of test_gpu_scan_groups.py: one launch of the chain per group, of the batch rows stated there."""
+    shapes = [(c[0], int(c[1] == torch.bfloat16), *c[2:8]) for c in GROUPS]
+    logs = _run(stub, f"""
+out = []
+for c in {shapes!r}:
+    stub.stub_reset()
+    assert call_mode(*c) == 0, c
+    out.append([op[2:] for op in log() if op[1] == "launch"])
+print(json.dumps(out))
+""")
+    for c, log in zip(GROUPS, logs):
+        chains = [int(op[2]) for op in log if "chain_fwd" in op[0] and "chain_fwd_reg" not in op[0]]
+        rows = [int(op[2]) for op in log if "rows_fwd" in op[0]]
+        B, H, group = c[2], c[4], c[8]
+        assert chains == rows == [H * min(group, B - b) for b in range(0, B, group)] and len(chains) > 1
+
+
+def test_projection_routes(stub):
+    """The few-row kernel runs while it has at most 512 workgroups, in the forward alone: the backward's products take the
+    tile kernels at every row count."""
+    most = [(256, 2048), (512, 1024), (2048, 256), (4096, 128), (8192, 64)]
+    shapes = [s for s, _ in FORWARD] + [(m, n, 96) for n, m in most] + [(m + 1, n, 96) for n, m in most]
+    want = [rows for _, rows in FORWARD] + [True] * len(most) + [False] * len(most)
+    fwd, bwd = _run(stub, f"""
+out = [[], []]
+p = 1 << 20
+for M, N, K in {shapes!r}:
+    stub.stub_reset()
+    assert lib.slotproj_fwd(p, p, p, M, N, K, p, None) == 0
+    out[0].append([op[2] for op in log()])
+for M, N, K in {BACKWARD!r}:
+    stub.stub_reset()
+    assert lib.slotproj_bwd(p, p, p, M, N, K, p, p, p, None) == 0
+    out[1].append([op[2] for op in log()])
+print(json.dumps(out))
+""")
+    assert [["proj_rows" in k for k in ks] for ks in fwd] == [[w] for w in want]
+    for ks in bwd:
+        assert [next(n for n in ("proj_transpose", "projt_gemm", "proj_gemm", "proj_reduce", "proj_rows") if n in k) for k in ks] \
+            == ["proj_transpose", "proj_gemm", "projt_gemm", "proj_reduce"]
