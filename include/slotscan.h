@@ -119,8 +119,10 @@ int slotscan_bwd_noalloc(const void* k, const void* q, const void* v, int dtype,
 /* Forward scan with the writer epilogue fused in.  Replaces kv_scan_g followed by the full-precision epilogue
  * of the writer layer (memlm_sh.py:453-456 then :473-475):
  *     nsq = kbuf.pow(2).sum(-1);  mem = (kbuf.to(bf16), vbuf.to(bf16), rsqrt(nsq.clamp_min(1e-12)), nsq > 1e-12)
- * The fp32 snapshots are never stored: the chain kernel emits each key snapshot row as bf16 together with
- * its kinv and valid, and the value replay emits each value snapshot row as bf16.
+ * The fp32 snapshots are never stored: the row replay (or, for many chains of a short scan, the chain kernel for its
+ * keys) emits each snapshot row as bf16, the keys' with kinv and valid.  The same outputs as slotscan_fwd_memq with
+ * bits = 0; without that call's key carry a long scan of few chains runs as one chunk, the replay behind the whole
+ * chain (B 8, T 1024, H 6, N 192, D 128: 652 us a call against 555).
  *   kb, vb   (B, ceil(T/G), H, N, D) bf16 (uint16 bit patterns)
  *   kinv     (B, ceil(T/G), H, N) fp32;  valid  (B, ceil(T/G), H, N) uint8 (0 / 1)
  * Every other argument is as in slotscan_fwd.  Applies where the epilogue follows the scan directly: not
@@ -156,8 +158,8 @@ int slotscan_bwd_mem(const void* k, const void* q, const void* v, int dtype,
  *     mem = (kq.to(bf16), _fq(vbuf, bits, group).to(bf16), rsqrt(nsq.clamp_min(1e-12)), nsq > 1e-12)
  * with _fq the midrise quantiser (memlm_sh.py:221-229; bits 2..8, one fp32 scale per `group` channels, a
  * power of two in [4, D]); bits = 0 emits the plain values (the same outputs as slotscan_fwd_mem).  The
- * chain kernel stores no key snapshots: the row replay rebuilds every key and value row from the address
- * log (bitwise the chain's state) and emits both copies.  run_sh25.sh:224 trains the last 20 % of its steps
+ * row replay rebuilds every key and value row from the address log (bitwise the chain's state) and emits both
+ * copies; with bits = 0 the chain kernel emits the keys' for many chains of a short scan.  run_sh25.sh:224 trains the last 20 % of its steps
  * this way (--qat_bits 3 --sh_qgroup 16).
  *   kcarry  (B*H, N, D) fp32 scratch in which the key replay carries its state across the forward
  *           pipeline's inner chunk boundaries: slotscan_fwd_carry_bytes(B, T, H, N, D, G) bytes, NULL when

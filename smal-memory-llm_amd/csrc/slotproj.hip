@@ -323,10 +323,12 @@ __global__ __launch_bounds__(64 * SWAVES) void proj_rows(ProjArgs p) {
     }
 }
 
-// out (M, N) = a w^T (+ d): proj_rows while its workgroups are at most two per CU, else proj_gemm.  Measured (us, proj_gemm
-// against proj_rows; N x K, rows): 2048 x 1536: 39 against 3.7 (1 row), 40 / 8.9 (64), 42 / 16 (256: 512 workgroups),
-// 42 / 32 (512), 43 / 66 (1,024); 512 x 512: 20 / 16 (1,024: 512), 20 / 31 (2,048); 2048 x 2048: 53 / 29 (256: 512),
-// 53 / 58 (512).
+// out (M, N) = a w^T (+ d), the forward: proj_rows while its workgroups are at most two per CU, else proj_gemm (the
+// backward's dRD always takes proj_gemm).  Both take time in proportion to K, which the rule leaves out; the line is
+// where no measured shape loses.  Measured (us, proj_gemm / proj_rows; N x K, rows): 2048 x 1536: 39 / 3.7 (1 row), 40 / 8.9
+// (64), 42 / 16 (256: 512 workgroups); 256 x 16384: 341 / 20 (1), 346 / 154 (2,048: 512); 512 x 512: 20 / 16 (1,024: 512); 2048 x
+// 2048: 53 / 29 (256: 512); 4096 x 4096: 94 / 45 (128: 512); 8192 x 1024: 31 / 16 (64: 512).  Beyond it the winner depends
+// on the shape: 2048 x 1536: 42 / 32 (512 rows), 43 / 66 (1,024); 512 x 512: 20 / 31 (2,048); 2048 x 2048: 53 / 58 (512).
 constexpr int64_t ROWS_MAX_WG = 512;
 static hipError_t launch_proj(const ProjArgs& a, hipStream_t st) {
     const unsigned nx = (unsigned)(a.N / 16);

@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(READ_THREADS) __attribute__((amdgpu_waves_per_eu(AC
 // qn = q / max(|q|, 1e-6) in bf16 and the multiplier exp(log_rsel) exp(C tanh(s / C)) of every read query, in one pass.
 // D / 8 lanes hold a query (16 bytes each), 256 lanes a workgroup: bound by its bytes (q in, qn out).  As torch
 // operations the same took seven passes and eleven launches forward and about fifteen backward; B 64, T 1024, H 6,
-// NQ 2, D 128, a reader layer's forward and backward: 4,390 us with them, 3,033 us with these.
+// NQ 2, D 128, a reader layer's forward and backward: 4,390 us with them, 3,061 us with these.
 struct PrepArgs {
     const bf16_t* q; const float* s; const float* log_rsel;
     const bf16_t* dqn; const float* dscale;              // backward: upstream gradients
@@ -1142,7 +1142,8 @@ __global__ __launch_bounds__(PREP_THREADS) void read_prep(PrepArgs a) {
 }
 
 // dq = dqn / nb - q [|q| >= 1e-6] <dqn, q> / (nb^2 |q|) (the norm's rounding to bf16 passes the gradient), in fp32 and
-// rounded once; ds = dscale scale (1 - tanh^2); the workgroup's sum of dscale scale for log_rsel.
+// rounded once, where the torch expressions round every intermediate result to bf16: dq's error against float64 (2-norm,
+// unit normal queries) is 2.3e-3 against their 2.9e-3, and the two differ by 2.9e-3; ds = dscale scale (1 - tanh^2); the workgroup's sum of dscale scale for log_rsel.
 template <int D>
 __global__ __launch_bounds__(PREP_THREADS) void read_prep_bwd(PrepArgs a) {
     constexpr int L = D / 8, RW = PREP_THREADS / L;

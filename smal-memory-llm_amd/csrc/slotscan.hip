@@ -699,10 +699,6 @@ template <int D, typename TI> struct ChainLds {
 };
 constexpr int FWD_THREADS = 256;
 
-// row-sized vectors at 4-byte aligned addresses (gfx950 takes dword-aligned vector accesses)
-typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
-typedef float f32x3u __attribute__((ext_vector_type(3), aligned(4)));
-
 template <int D, int NR, typename TI, bool LOG>
 __global__ __attribute__((amdgpu_flat_work_group_size(FWD_THREADS, FWD_THREADS), amdgpu_waves_per_eu(1)))
 void chain_fwd(ChainFwdArgs a) {
@@ -907,7 +903,7 @@ void chain_fwd(ChainFwdArgs a) {
         const float temp = a.temp[0];
         const float eps = a.eps;
         const bool occb = a.occb != 0;
-        // this lane's rows: n0 .. n0 + NR - 1 (one vector store per step logs their cosines)
+        // this lane's rows: n0 .. n0 + NR - 1 (a step leaves their cosines in their records, in place of its scores)
         const int n0 = NR * lane;
         // the rows that compete: occupied ones and the lowest free one
         auto compete = [&]() __attribute__((always_inline)) {
@@ -3000,7 +2996,7 @@ struct FwdOut {
     int8_t* kcode; float* kscale; int8_t* vcode; float* vscale;
     int bits, group;
     float* kcarry;                                       // FE_MEM / FE_CODES: the key replay's chunk carry
-    bool one;                                            // no carry to hand: one chunk
+    bool one;                                            // no carry to hand (slotscan_fwd_mem): one chunk
 };
 
 // chunk length of the forward pipeline (a multiple of G); T < 512 runs as one chunk
@@ -3009,11 +3005,15 @@ static int64_t fwd_chunk_len(int64_t T, int64_t G) {
 }
 
 // The forward pipeline's chunk boundaries b[0] = 0 < b[1] < ... < b[n] = T (inner ones multiples of G);
-// returns n (at most FWD_MAX_CHUNKS).  Equal chunks of fwd_chunk_len, unless the value replay fits one round
-// of workgroups (two per CU): it then takes well under half the chain's time per step (the chain is bound
-// by its step latency), and the chunks halve towards the end (..., 128, 64, 32, 32 steps at G = 8), so that
-// the tail the replay leaves exposed (the last chunk's) and the number of chunk starts are both small, while
-// each replay still hides behind the next chain chunk, half as long.
+// returns n (at most FWD_MAX_CHUNKS).  Equal chunks of fwd_chunk_len, unless the row replay fits one round
+// of workgroups (two per CU): then the chunks halve towards the end (..., 128, 64, 32, 32 steps at G = 8), so that
+// the tail the replay leaves exposed (the last chunk's) and the number of chunk starts are both small; a replay
+// hides behind the next chain chunk, half as long, where it takes at most half of the chain's time per step.
+// At N 192, D 128, H 6 a step of the chain takes 0.45 us and one of the replay, for 48 chains, 0.20 (bf16 copies), 0.27
+// (fp32), 0.28 (codes) or 0.34 us (quantised copies), for 84 chains 0.26, 0.41, 0.31 or 0.38.  T 1,024, us with halving /
+// equal chunks: 48 chains, bf16 copies 536 / 581, fp32 553 / 592, codes 586 / 595, quantised 649 / 608; 84 chains, bf16
+// copies 555 / 600, codes 624 / 610, fp32 688 / 622, quantised 689 / 624.  So where the replay takes more than half, equal
+// chunks would be the better ones; the line here does not count that.
 #define FWD_MAX_CHUNKS 40
 static_assert(FWD_MAX_CHUNKS <= slothost::FORK_EVENTS, "a forward holds an event per chunk");
 static int fwd_chunks(int64_t B, int64_t T, int64_t H, int64_t N, int64_t G, int64_t* b) {
@@ -3027,7 +3027,7 @@ static int fwd_chunks(int64_t B, int64_t T, int64_t H, int64_t N, int64_t G, int
     }
     // on the whole blocks of T (the last chunk takes T % G too): the tail m, m, 2m, 4m, ... from the end while
     // the rest is at least twice the next size, then the rest as one chunk, or two if it is over twice the tail's
-    // largest (a replay runs at well under half its chain's time per step, so each hides behind the next chunk)
+    // largest
     const int64_t Tg = (T / G) * G;
     const int64_t m = ((std::max<int64_t>(32, G) + G - 1) / G) * G;
     int64_t tail[FWD_MAX_CHUNKS];

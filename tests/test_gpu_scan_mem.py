@@ -1,5 +1,5 @@
 """GPU parity of the fused scan + writer epilogue (slotkern_hip.kv_scan_mem, libslotscan.so's
-slotscan_fwd_mem / slotscan_bwd_mem) -- the writer layer's kv_scan_g followed by its full-precision
+slotscan_fwd_memq with slotscan_bwd_mem, or with bits > 0 slotscan_bwd_memq) -- the writer layer's kv_scan_g followed by its full-precision
 epilogue (memlm_sh.py:453-456, 473-475).
 
 Two references on the same seeded inputs:
