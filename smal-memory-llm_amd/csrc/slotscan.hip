@@ -3012,7 +3012,7 @@ static int64_t fwd_chunk_len(int64_t T, int64_t G) {
 // At N 192, D 128, H 6 a step of the chain takes 0.45 us and one of the replay, for 48 chains, 0.20 (bf16 copies), 0.27
 // (fp32), 0.28 (codes) or 0.34 us (quantised copies), for 84 chains 0.26, 0.41, 0.31 or 0.38.  T 1,024, us with halving /
 // equal chunks: 48 chains, bf16 copies 536 / 581, fp32 553 / 592, codes 586 / 595, quantised 649 / 608; 84 chains, bf16
-// copies 555 / 600, codes 624 / 610, fp32 688 / 622, quantised 689 / 624.  So where the replay takes more than half, equal
+// copies 555 / 600, codes 624 / 610, fp32 688 / 622 (T 4,096: 2,798 / 2,196), quantised 689 / 624.  So where the replay takes more than half, equal
 // chunks would be the better ones; the line here does not count that.
 #define FWD_MAX_CHUNKS 40
 static_assert(FWD_MAX_CHUNKS <= slothost::FORK_EVENTS, "a forward holds an event per chunk");
