@@ -1210,12 +1210,10 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
 #pragma unroll
                 for (int e = 0; e < EPL; e++) { kv[e] = K[e]; vv[e] = V[e]; }
             }
-            if (KR) {
-                float sq = 0.f;
+            float sq = 0.f;
 #pragma unroll
-                for (int e = 0; e < EPL; e++) sq = fmaf(kv[e], kv[e], sq);
-                ks[0] = rowsum16(sq);
-            }
+            for (int e = 0; e < EPL; e++) sq = fmaf(kv[e], kv[e], sq);
+            ks[0] = rowsum16(sq);
 #pragma unroll
             for (int jj = 0; jj < NP; jj++) {
                 kx[jj] = u32x2{pack_bf16x2(kv[4 * jj], kv[4 * jj + 1]), pack_bf16x2(kv[4 * jj + 2], kv[4 * jj + 3])};
@@ -1228,7 +1226,7 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
                     const u32x2 rcv = {dppu<SLOT_DPP_XOR1>(snd.x), dppu<SLOT_DPP_XOR1>(snd.y)};
                     if (odd) x[0] = rcv; else x[1] = rcv;
                 };
-                if (KR) trade(kx);
+                trade(kx);
                 trade(vx);
             }
         }
@@ -1254,9 +1252,9 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
                 if constexpr (NP == 2) __builtin_nontemporal_store(u32x4{x[0].x, x[0].y, x[NP - 1].x, x[NP - 1].y}, reinterpret_cast<u32x4*>(r));
                 else __builtin_nontemporal_store(x[0], reinterpret_cast<u32x2*>(r));
             };
-            if (KR) put(a.kbm, kx);
+            put(a.kbm, kx);
             put(a.vbm, vx);
-            if (KR && c == 0) {                                // kinv and valid of the emitted (quantised) keys
+            if (c == 0) {                                // kinv and valid of the emitted (quantised) keys
                 a.kinvm[srow] = rsqrtf(fmaxf(ks[0], 1e-12f));
                 a.validm[srow] = ks[0] > 1e-12f ? 1 : 0;
             }
@@ -1294,6 +1292,8 @@ ROWS_ATTR void rows_fwd(RowsFwdArgs a) {
                             if (KR) st_slice_nt<EPL>(a.kbuf + srow * D, K, c);
                             st_slice_nt<EPL>(a.vbuf + srow * D, V, c);
                         }
+                    } else if constexpr (EM == RF_MEMV) {   // (short scans: holding and 16-byte stores cost 13-16 %)
+                        st_slice_bf_at<EPL>(a.vbm + srow * D, 8u * (u32)c, V);
                     } else {
                         if (!fresh) { form(); fresh = true; }
                         emit();
@@ -3097,7 +3097,7 @@ static bool fwd_chain_reg(int mode, int bits, int64_t chains, int64_t Tc, int64_
         else lim = wide ? 16 : 8;
     } else if (full && wide) {                           // as many rounds: only the start is longer
         lim = f32 ? (Tc > 8 || rn > 4 ? 32 : 0) : rn == 1 ? 0 : mem ? 4 : 8;
-    } else if (full && f32 && D == 128 && rn > 1) {
+    } else if (full && D == 128 && (f32 ? rn > 1 : mem && rn > 4)) {
         lim = 4;
     }
     return Tc <= lim;

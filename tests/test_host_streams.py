@@ -171,7 +171,7 @@ def test_register_chain_cases_take_it(stub):
     ("f32", 1, 256, 192, 128, 0), ("f32", 1, 264, 192, 128, 4096), ("f32", 1, 4096, 96, 128, 4), ("f32", 0, 1024, 96, 128, 64),
     ("f32", 0, 512, 192, 64, 128), ("f32", 0, 1024, 192, 64, 96), ("f32", 1, 1024, 96, 64, 32), ("f32", 1, 4096, 64, 128, 0),
     ("mem", 1, 256, 192, 128, 0), ("mem", 1, 264, 192, 128, 64), ("mem", 1, 512, 192, 128, 96), ("mem", 1, 4096, 192, 128, 48),
-    ("mem", 1, 1024, 128, 128, 16), ("mem", 1, 768, 128, 128, 8), ("mem", 0, 768, 192, 64, 16), ("mem", 1, 1024, 96, 64, 8),
+    ("mem", 1, 4096, 96, 128, 4), ("mem", 1, 1024, 128, 128, 16), ("mem", 1, 768, 128, 128, 8), ("mem", 0, 768, 192, 64, 16), ("mem", 1, 1024, 96, 64, 8),
     ("memq", 1, 1024, 192, 128, 16), ("codes", 1, 1024, 192, 128, 16), ("codes", 1, 1024, 128, 128, 8), ("codes", 1, 4096, 96, 128, 0),
 ])
 def test_register_chain_rule(stub, mode, bf16, chains, N, D, longest):
